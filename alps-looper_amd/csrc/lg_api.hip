@@ -239,6 +239,25 @@ static long long op_capacity(const lg_params& p, const ChainDev& d) {
   return (long long)std::ceil(bound + 10.0 * std::sqrt(bound) + 1024.0);
 }
 
+// expected operators of a chain: per bond beta * (offset + half the largest
+// diagonal energy), site operators beta |hx|
+static double expected_ops(const lg_params& p, const ChainDev& d) {
+  const double per_bond = (d.offset_total - d.N * d.site_w) / d.nb_real +
+                          0.5 * (std::fabs(p.jz) / 4 + std::fabs(p.jxy) / 2);
+  return d.beta * (d.nb_real * per_bond + d.N * 2 * d.site_w);
+}
+
+// Time of a sweep (us): a chain in one workgroup, and a batch on the flat
+// kernels.  Fitted to chains of 41 to 24000 operators on 16 to 3072 bonds
+// (one workgroup: 18 us at 41 operators, 22 at 450, 65 at 3000 on 512 bonds,
+// 40 at 350 on 2048, 540 at 24000 on 2048, where the clusters' accumulators
+// take several passes) and on the flat kernels' launches (65 us at 450
+// operators, 83 at 8900, 140 with virtual sites, 1050 at 3.2M in 512 chains).
+static double block_us(double n, int bonds) {
+  return 14.0 + 0.016 * n + 0.012 * bonds + 0.01 * std::max(0.0, n - 12000.0);
+}
+static double flat_us(double n, bool general) { return (general ? 120.0 : 70.0) + 0.00035 * n; }
+
 // ---------------------------------------------------------------------------
 // Batch
 // ---------------------------------------------------------------------------
@@ -353,6 +372,7 @@ int Batch::init_exchange(const lg_params& p, const double* betas, int n, uint32_
   }
   Capacity cap;
   cap.chains = n;
+  long long ops_max = 0;
   for (int t = 0; t < n; ++t) {
     ds[t].cand_cap = cand_cap;
     Footprint f = footprint(ps[t]);
@@ -360,6 +380,13 @@ int Batch::init_exchange(const lg_params& p, const double* betas, int n, uint32_
     cap.bonds += f.bonds;
     cap.ops += f.ops;
     cap.cand += (long long)ds[t].Nb * cand_cap;
+    ops_max = std::max(ops_max, f.ops);
+  }
+  // one workgroup per chain keeps every chain in a region of its own, which
+  // has to hold the largest beta's operators
+  if (n * ops_max <= (1ll << 26)) {
+    blk_exchange_ops = ops_max;
+    cap.ops = std::max(cap.ops, n * ops_max);
   }
   if ((rc = reserve(cap, false))) return rc;
   params = ps;
@@ -379,6 +406,7 @@ int Batch::init_exchange(const lg_params& p, const double* betas, int n, uint32_
   LG_HIP(hipMemset(xacc, 0, (n - 1) * sizeof(unsigned long long)));
   LG_HIP(hipMemset(xstep, 0, sizeof(uint32_t)));
   nslots = n;
+  if (blk_exchange_ops == 0) blk_fit = false;
   xkey0 = seed;
   xkey1 = 0xffffffffu;
   invalidate_graphs();
@@ -434,10 +462,10 @@ int Batch::reserve(const Capacity& cap, bool dynamic) {
   node_cap = (int)ncap;
   cand_total = cap.cand;
   LG_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  return allocate();
+  return allocate(dynamic);
 }
 
-int Batch::allocate() {
+int Batch::allocate(bool dynamic) {
   int rc = 0;
   for (int i = 0; i < 2; ++i) {
     State& s = st[i];
@@ -480,6 +508,9 @@ int Batch::allocate() {
   if ((rc = alloc(scan_ctl, 2))) return rc;
   LG_HIP(hipMemset(scan_status, 0, scan_nparts * sizeof(unsigned long long)));
   LG_HIP(hipMemset(scan_ctl, 0, 2 * sizeof(int)));
+  // one workgroup per chain, except for server batches, whose mixes hold jobs
+  // too large for it and whose sweeps replay the graph of each layout
+  blk_lds_grant = !dynamic && block_prepare() ? BLOCK_LDS_MAX : 0;
   if ((rc = alloc(col_part, (size_t)col_chunks(node_cap) * NUM_COLLECTOR_TERMS))) return rc;
   if ((rc = alloc(totals, 2))) return rc;
   if ((rc = alloc(flags, 1))) return rc;
@@ -564,6 +595,7 @@ int Batch::set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sw
   nsites = (int)sites;
   nbonds = (int)bonds;
   host_sweep = sweeps;
+  choose_block();
   std::vector<int> bc(std::max(nbonds, 1)), sc(std::max(nsites, 1));
   std::vector<uint32_t> sw(std::max<size_t>(chains.size(), 1));
   for (size_t c = 0; c < chains.size(); ++c) {
@@ -648,6 +680,124 @@ int Batch::set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sw
   return apply_cfg(c);
 }
 
+// Regions of the chains, and whether the batch takes one workgroup per chain.
+void Batch::choose_block() {
+  blk_fit = false;
+  const size_t nc = chains.size();
+  if (nc == 0 || is_sse() || blk_lds_grant <= 0) return;
+  double most = 0, longest = 0, sum = 0, total = 0;
+  long long ops = 0, nodes = 0;
+  int lds = 0, least = 0;
+  bool general = false;
+  std::vector<std::pair<double, int>> order(nc);
+  for (size_t c = 0; c < nc; ++c) {
+    ChainDev& d = chains[c];
+    // (site pairs in 16 + 16 bits, candidate ranks in 10, tables in LDS)
+    if (d.N > 0xffff || d.Nb > 16384 || d.cand_cap > 1024) return;
+    // operators of a chain's region: a replica of an exchange may come to the
+    // largest beta, one chain has the whole capacity
+    long long cap = nc == 1 ? op_cap : footprint(params[c]).ops;
+    if (blk_exchange_ops > 0) cap = blk_exchange_ops;
+    const long long ncap = 2 * cap + d.N;
+    if (ops + cap > op_cap || nodes + ncap > node_cap) return;
+    d.blk_op = (int)ops;
+    d.blk_node = (int)nodes;
+    d.blk_opcap = (int)cap;
+    d.blk_nodecap = (int)ncap;
+    ops += cap;
+    nodes += ncap;
+    const double n = expected_ops(params[c], d);
+    if (n > 1.0e5) return;
+    order[c] = {n, (int)c};
+    most = std::max(most, n);
+    const double us = block_us(n, d.Nb);
+    longest = std::max(longest, us);
+    sum += us;
+    total += n;
+    least = std::max(least, block_lds_least(d));
+    lds = std::max(lds, block_lds_for(d, (int)(1.1 * n) + 64));
+    general = general || d.nv > 1 || d.Nb > d.nb_lat;
+  }
+  if (least > blk_lds_grant) return;
+  blk_lds = std::min(std::max(lds, least), blk_lds_grant);
+  blk_threads = most <= 256 ? 256 : (most <= 1024 ? 512 : 1024);
+  blk_general = general;
+  // a batch lasts as long as its longest chain, or as its chains over the CUs
+  blk_us = std::max(longest, sum / std::max(cus, 1));
+  if (blk_us > flat_us(total, general)) return;
+  std::sort(order.begin(), order.end(), [](const auto& x, const auto& y) { return x.first != y.first ? x.first > y.first : x.second < y.second; });
+  std::vector<int> idx(nc);
+  for (size_t i = 0; i < nc; ++i) idx[i] = order[i].second;
+  // its buffers, once (the order, and k_pack's bases; counts; segment scratch)
+  if (!blk_info && (alloc(blk_order, 3 * (size_t)cap_chains) || alloc(blk_nops, cap_chains) || alloc(blk_nnodes, cap_chains) ||
+                     alloc(blk_root, node_cap) || alloc(blk_len, node_cap) || alloc(blk_info, node_cap)))
+    return;
+  if (hipMemcpy(blk_order, idx.data(), nc * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) return;
+  blk_fit = true;
+}
+
+// n sweeps with one workgroup per chain, records to the ring from slot0 on.
+// A launch takes as many sweeps as fit about 20 ms, so that other streams'
+// work is not held up; a replica exchange comes after every sweep.
+int Batch::run_block(uint32_t n, uint32_t slot0) {
+  const uint32_t most = nslots > 1 ? 1u : (uint32_t)std::max(1.0, std::min(4096.0, 20000.0 / blk_us));
+  for (uint32_t done = 0; done < n;) {
+    // out of the packed form one sweep by itself: a second one would write
+    // this chain's region of the arrays in which a chain whose workgroup has
+    // not started yet still has its configuration
+    const bool leave_packed = !blk_regions && chains.size() > 1;
+    const uint32_t k = leave_packed ? 1u : std::min(n - done, most);
+    DevBatch B = dev(cur);
+    BlockArgs A;
+    A.order = blk_order;
+    A.grid = (int)chains.size();
+    A.nsweeps = (int)k;
+    A.slot0 = (int)(slot0 + done);
+    A.lds = blk_lds;
+    A.packed = blk_regions ? 0 : 1;
+    A.nops = blk_nops;
+    A.nnodes = blk_nnodes;
+    A.root_of = blk_root;
+    A.seg_len = blk_len;
+    A.seg_info = blk_info;
+    launch_chain_sweeps(B, A, blk_general, blk_threads, stream);
+    if (nslots > 1) {
+      B.blk_nops = blk_nops;
+      launch_exchange(B, stream);
+    }
+    LG_HIP(hipGetLastError());
+    if (k & 1) cur ^= 1;
+    blk_regions = chains.size() > 1;
+    note_swept();
+    done += k;
+  }
+  return LG_OK;
+}
+
+int Batch::ensure_packed() {
+  if (!blk_regions) return LG_OK;
+  const size_t nc = chains.size();
+  std::vector<int> n(nc), m(nc), base(2 * nc);
+  LG_HIP(hipStreamSynchronize(stream));
+  LG_HIP(hipMemcpy(n.data(), blk_nops, nc * sizeof(int), hipMemcpyDeviceToHost));
+  LG_HIP(hipMemcpy(m.data(), blk_nnodes, nc * sizeof(int), hipMemcpyDeviceToHost));
+  long long ops = 0, nodes = 0;
+  for (size_t c = 0; c < nc; ++c) {
+    base[c] = (int)ops;
+    base[nc + c] = (int)nodes;
+    ops += n[c];
+    nodes += m[c];
+  }
+  int* const d_base = blk_order + cap_chains;
+  LG_HIP(hipMemcpy(d_base, base.data(), 2 * nc * sizeof(int), hipMemcpyHostToDevice));
+  launch_pack(dev(cur), blk_nops, blk_nnodes, d_base, d_base + nc, stream);
+  LG_HIP(hipGetLastError());
+  LG_HIP(hipStreamSynchronize(stream));
+  cur ^= 1;
+  blk_regions = false;
+  return LG_OK;
+}
+
 int Batch::apply_cfg(const LaunchCfg& c) {
   // the compress pass clears the roots' accumulators before the estimator
   // adds into them; without it they must be zero between sweeps, which the
@@ -662,6 +812,7 @@ int Batch::apply_cfg(const LaunchCfg& c) {
 // all-up spins, empty operator string (path_integral.C:225) for every chain
 int Batch::reset_state() {
   cur = 0;
+  blk_regions = false;
   State& s = st[cur];
   std::vector<int> zeros(nbonds + 1, 0), soff(nsites + 1);
   for (int i = 0; i <= nsites; ++i) soff[i] = i;
@@ -793,6 +944,7 @@ DevBatch Batch::dev(int from) const {
   B.sse_new = sse_str[1 - from];
   B.sse_perm = kpre;  // (the path-integral diagonal update's, unused by SSE batches)
   B.sched = d_sched;
+  B.blk_nops = nullptr;
   return B;
 }
 
@@ -853,13 +1005,19 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
   if (rc) return rc;
   const size_t nc = chains.size();
   if (nc == 0) return LG_OK;
+  const bool block = block_form();
+  if (!block && (rc = ensure_packed())) return rc;
   uint32_t done = 0;
   while (done < n) {
     uint32_t chunk = std::min<uint32_t>(n - done, (uint32_t)ring_size);
-    LG_HIP(hipMemsetAsync(ring_pos, 0, sizeof(int), stream));
-    for (uint32_t i = 0; i < chunk; ++i) {
-      rc = enqueue_sweep();
-      if (rc) return rc;
+    if (block) {
+      if ((rc = run_block(chunk, 0))) return rc;
+    } else {
+      LG_HIP(hipMemsetAsync(ring_pos, 0, sizeof(int), stream));
+      for (uint32_t i = 0; i < chunk; ++i) {
+        rc = enqueue_sweep();
+        if (rc) return rc;
+      }
     }
     const size_t words = (size_t)chunk * nc * R_COUNT;
     if (out) LG_HIP(hipMemcpyAsync(rec_host, rec_ring, words * sizeof(double), hipMemcpyDeviceToHost, stream));
@@ -881,8 +1039,18 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
 // live configuration.
 int Batch::tune(uint32_t sweeps_per_trial) {
   if (sweeps_per_trial == 0) sweeps_per_trial = 8;
-  int rc = run(sweeps_per_trial, nullptr);  // warm state and code
+  // the first trial warms state and code, and times one workgroup per chain
+  // (after its first sweep) where the batch can take it
+  blk_off = false;
+  int rc = run(1, nullptr);
   if (rc) return rc;
+  double block_t = blk_us * 1e-6;
+  if (sweeps_per_trial > 1) {
+    const auto t0 = std::chrono::steady_clock::now();
+    if ((rc = run(sweeps_per_trial - 1, nullptr))) return rc;
+    block_t = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() / (sweeps_per_trial - 1);
+  }
+  blk_off = true;
   LaunchCfg best = cfg;
   double best_t = 1e300;
   const int groups[] = {1, 2, 4, 8, 16, 32, 64};
@@ -918,6 +1086,7 @@ int Batch::tune(uint32_t sweeps_per_trial) {
     }
   }
   tuned = true;
+  blk_off = !blk_fit || block_t > best_t / sweeps_per_trial;
   return apply_cfg(best);
 }
 
@@ -961,6 +1130,7 @@ int Batch::set_launch(const lg_launch& l) {
     c.est_flush = l.flush;
   }
   tuned = true;
+  blk_off = true;  // the given settings are the flat kernels'
   return apply_cfg(c);
 }
 
@@ -970,9 +1140,31 @@ int Batch::profile(uint32_t n, double* ms) {
   int rc = check_flags();
   if (rc) return rc;
   const int K = NUM_SWEEP_KERNELS;
+  for (int i = 0; i < NUM_PROFILED; ++i) ms[i] = 0;
+  if (block_form()) {  // one workgroup per chain: the launches as a whole
+    hipEvent_t e0, e1;
+    LG_HIP(hipEventCreate(&e0));
+    LG_HIP(hipEventCreate(&e1));
+    for (uint32_t done = 0; done < n;) {
+      const uint32_t chunk = std::min<uint32_t>(n - done, (uint32_t)ring_size);
+      LG_HIP(hipEventRecord(e0, stream));
+      if ((rc = run_block(chunk, 0))) return rc;
+      LG_HIP(hipEventRecord(e1, stream));
+      LG_HIP(hipStreamSynchronize(stream));
+      float t = 0;
+      LG_HIP(hipEventElapsedTime(&t, e0, e1));
+      ms[NUM_SWEEP_KERNELS] += t;
+      done += chunk;
+      for (size_t c = 0; c < chains.size(); ++c) host_sweep[c] += chunk;
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    ms[NUM_SWEEP_KERNELS] /= std::max<uint32_t>(n, 1);
+    return check_flags();
+  }
+  if ((rc = ensure_packed())) return rc;
   std::vector<hipEvent_t> ev((size_t)(K + 1) * std::max<uint32_t>(n, 1));
   for (auto& e : ev) LG_HIP(hipEventCreate(&e));
-  for (int i = 0; i < K; ++i) ms[i] = 0;
   uint32_t done = 0;
   while (done < n) {
     uint32_t chunk = std::min<uint32_t>(n - done, (uint32_t)ring_size);
@@ -1144,6 +1336,12 @@ int Batch::get_config(int c, int32_t* spins, int32_t* bond_offsets, double* time
 }
 
 int Batch::num_ops(int c, long long* n) {
+  if (blk_regions) {
+    int v = 0;
+    LG_HIP(hipMemcpy(&v, blk_nops + c, sizeof(int), hipMemcpyDeviceToHost));
+    *n = v;
+    return LG_OK;
+  }
   const ChainDev& d = chains[c];
   int a = 0, b = 0;
   LG_HIP(hipMemcpy(&a, st[cur].bo + d.bond_base, sizeof(int), hipMemcpyDeviceToHost));
@@ -1158,6 +1356,7 @@ int Batch::chain_config(int c, std::vector<int>& spins, std::vector<int>& bo, st
   if (!swept_since_layout && (chains[c].old_site_base != chains[c].site_base ||
                               chains[c].old_bond_base != chains[c].bond_base))
     return set_error(LG_ERR_STATE, "chain moved since its last sweep");
+  if (int rc = ensure_packed()) return rc;
   LG_HIP(hipStreamSynchronize(stream));
   const ChainDev& d = chains[c];
   const State& s = st[cur];
@@ -1181,6 +1380,7 @@ int Batch::chain_config(int c, std::vector<int>& spins, std::vector<int>& bo, st
 
 int Batch::load_configs(const std::vector<HostConfig>& cfg) {
   if (cfg.size() != chains.size()) return set_error(LG_ERR_ARG, "one configuration per chain");
+  blk_regions = false;
   std::vector<uint8_t> sp(std::max(nsites, 1));
   std::vector<int> bo(nbonds + 1), soff(nsites + 1);
   std::vector<double> ot, evt;
@@ -1784,10 +1984,10 @@ int lg_copy_bandwidth(uint64_t bytes, int iters, double* gbs) {
   return LG_OK;
 }
 
-int lg_profile_num_kernels(void) { return lg::NUM_SWEEP_KERNELS; }
+int lg_profile_num_kernels(void) { return lg::NUM_PROFILED; }
 
 const char* lg_profile_kernel_name(int i) {
-  return (i >= 0 && i < lg::NUM_SWEEP_KERNELS) ? lg::kKernelNames[i] : "";
+  return (i >= 0 && i < lg::NUM_PROFILED) ? lg::kKernelNames[i] : "";
 }
 
 int lg_chain_profile(lg_chain* h, uint32_t n, double* avg_ms) {

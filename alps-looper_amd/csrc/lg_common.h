@@ -98,6 +98,9 @@ struct ChainDev {
   // (antiferromagnetic XY) and on the site bonds (hx < 0); the
   // configuration's sign is (-1)^(their number)
   int sgn_lattice, sgn_site;
+  // one workgroup per chain (lg_block.hip): the chain's own regions of the
+  // operator and segment arrays
+  int blk_op, blk_node, blk_opcap, blk_nodecap;
 };
 // SSE chains: their sites' spins and bonds' counters are staged in LDS
 constexpr int SSE_MAX_SITES = 4096, SSE_MAX_BONDS = 4096;

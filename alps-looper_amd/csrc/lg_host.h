@@ -108,6 +108,8 @@ class Batch {
                    int32_t* types_out, int64_t* n_clusters);
   DevBatch dev(int from) const;
   int enqueue_sweep();
+  // the next run takes one workgroup per chain (lg_block.hip)
+  bool block_form() const { return blk_fit && !blk_off; }
 
   std::vector<lg_params> params;
   std::vector<ChainDev> chains;
@@ -139,7 +141,7 @@ class Batch {
   // new bases (contiguous in the given order), chain tables, sweep counters;
   // check_old: also check the previous bases a relayout leaves the chains with
   int set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sweeps, bool check_old = false);
-  int allocate();
+  int allocate(bool dynamic);
   int reset_state();
   void release();
   void invalidate_graphs();
@@ -147,6 +149,10 @@ class Batch {
   int apply_cfg(const LaunchCfg& c);
   int capture(int from);
   int check_flags();
+  void choose_block();
+  int run_block(uint32_t n, uint32_t slot0);
+  // st[cur] in the packed form (the chains' operators and segments consecutive)
+  int ensure_packed();
   void note_swept();
 
   std::vector<void*> allocations;
@@ -195,6 +201,19 @@ class Batch {
   unsigned long long* xacc = nullptr;
   uint32_t* xstep = nullptr;
   uint32_t xkey0 = 0, xkey1 = 0;
+  // one workgroup per chain (lg_block.hip): every chain fits and it is the
+  // faster form (blk_fit), unless launch settings were given (blk_off);
+  // blk_regions: st[cur] stands in the chains' own regions
+  bool blk_fit = false, blk_off = false, blk_regions = false, blk_general = false;
+  int blk_lds = 0, blk_threads = 0, blk_lds_grant = 0;
+  double blk_us = 0;            // expected time of a sweep
+  long long blk_exchange_ops = 0;  // operators of a region of an exchange batch
+  int* blk_order = nullptr;
+  int* blk_nops = nullptr;
+  int* blk_nnodes = nullptr;
+  int* blk_root = nullptr;
+  double* blk_len = nullptr;
+  uint32_t* blk_info = nullptr;
   // annealing schedules (one chain): table of (start step, temperature) pairs
   std::vector<double> sched_host;
   double* d_sched = nullptr;

@@ -88,6 +88,22 @@ struct DevBatch {
   const int* sse_old;          // operator strings of the previous configuration (ChainDev::sse_base)
   int* sse_new;                // operator strings being built
   int* sse_perm;               // [ops] string position -> operator index of the new configuration
+  const int* blk_nops;         // [nchains] operators per chain when each stands in its own region (else null)
+};
+
+// one workgroup per chain (lg_block.hip)
+struct BlockArgs {
+  const int* order;    // [grid] chain of each workgroup
+  int grid;
+  int nsweeps;         // sweeps of this launch; with an even number the last configuration is in the "old" arrays
+  int slot0;           // ring slot of its first sweep
+  int lds;             // LDS bytes of a workgroup
+  int packed;          // the previous configuration is in the packed form (offsets of consecutive chains meet)
+  int* nops;           // [chains] operators and segments of a chain's configuration
+  int* nnodes;
+  int* root_of;        // [nodes] root segment of each cluster
+  double* seg_len;     // [nodes] a segment's length, and its cluster, class, tau = 0 and winding terms
+  uint32_t* seg_info;
 };
 
 struct LaunchCfg {
@@ -110,7 +126,9 @@ struct LaunchCfg {
 
 constexpr int NUM_SWEEP_KERNELS = 9;
 constexpr int NUM_COLLECTOR_TERMS = 19;   // per-cluster terms summed into the sweep record
-extern const char* const kKernelNames[NUM_SWEEP_KERNELS];
+// the profiled kernels: the flat sweep's, then the sweep by one workgroup per chain
+constexpr int NUM_PROFILED = NUM_SWEEP_KERNELS + 1;
+extern const char* const kKernelNames[NUM_PROFILED];
 
 void launch_sweep(const DevBatch& B, const LaunchCfg& L, hipStream_t st, hipEvent_t* ev = nullptr);
 void launch_cluster_stage(const DevBatch& B, const LaunchCfg& L, hipStream_t st, hipEvent_t* ev = nullptr);
@@ -118,6 +136,15 @@ void launch_site_scan(const DevBatch& B, hipStream_t st);
 void launch_canon(const DevBatch& B, int chain, int nelem, int* canon, int* labels, int* roots,
                   hipStream_t st);
 int scan_blocks(const DevBatch& B);
+// LDS that a workgroup of k_chain_sweeps can ask for (160 KB less its static part)
+constexpr int BLOCK_LDS_MAX = 160 * 1024 - 4096;
+int block_prepare();                          // 1 when the device grants that much
+int block_lds_least(const ChainDev& d);       // the least that serves any configuration of a chain's region
+int block_lds_for(const ChainDev& d, int n);  // with n operators, every step's arrays at once
+void launch_chain_sweeps(const DevBatch& B, const BlockArgs& A, bool general, int threads, hipStream_t st);
+void launch_pack(const DevBatch& B, const int* nops, const int* nnodes, const int* op_base, const int* node_base,
+                 hipStream_t st);
+void launch_exchange(const DevBatch& B, hipStream_t st);
 int col_chunks(int node_cap);
 
 }  // namespace lg

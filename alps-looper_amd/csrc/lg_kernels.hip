@@ -28,6 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include "lg_common.h"
+#include "lg_device.h"
 #include "lg_kernels.h"
 
 namespace lg {
@@ -35,8 +36,6 @@ namespace lg {
 // ---------------------------------------------------------------------------
 // small helpers
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
-
 template <int G>
 __device__ __forceinline__ int glane() { return threadIdx.x & (G - 1); }
 
@@ -118,10 +117,6 @@ __device__ __forceinline__ void xcd_share(int n, int& lo, int& hi) {
   const long long s1 = (long long)n * ((x + 1) * q + min(x + 1, r)) / nb;
   lo = (int)(s0 + (s1 - s0) * j / nbx);
   hi = (int)(s0 + (s1 - s0) * (j + 1) / nbx);
-}
-
-__device__ __forceinline__ bool overflowed(const DevBatch& B) {
-  return __hip_atomic_load(B.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
 // chain of a segment node by binary search over the chains' first nodes
@@ -1208,26 +1203,7 @@ __global__ void __launch_bounds__(256) k_uf_union(DevBatch B) {
   }
 }
 
-// tau boundary of the virtual sites (S > 1/2; path_integral.C:589-615, the
-// S > 1/2 branch of the symmetrization): per real site, the tau = 0 ends
-// (lowest segments) of its nv virtual sites are joined to their tau = 1 ends
-// (top segments) by a permutation that maps equal spins onto each other,
-// uniform among those that do (looper::partitioned_random_shuffle,
-// looper/permutation.h:88-112).  For each spin value u = 0, 1 in turn, the
-// bottoms of spin u in virtual-site order are matched to the tops of spin u
-// in virtual-site order permuted by Fisher-Yates: for i = n_u - 1 down to 1,
-// j = i - (x mod (i + 1)) with x the next word of the stream (word k is word
-// k mod 4 of Philox(sweep, STAGE_BOUNDARY, real site, k / 4)), swap
-// positions i and j.  (The spins at tau = 1 are those at tau = 0 in some
-// order: every update keeps each real site's magnetization periodic.)  For
-// nv = 2 with equal spins this is the exchange iff bit 0 of the first word
-// is set.  One thread per real site; nv <= 8, so a permutation lives in one
-// register as eight 4-bit fields.
-template <typename T>
-__device__ __forceinline__ T pick8(int i, T a0, T a1, T a2, T a3, T a4, T a5, T a6, T a7) {
-  return i < 4 ? (i == 0 ? a0 : i == 1 ? a1 : i == 2 ? a2 : a3) : (i == 4 ? a4 : i == 5 ? a5 : i == 6 ? a6 : a7);
-}
-
+// tau boundary of the virtual sites (join_boundary), one thread per real site
 __global__ void __launch_bounds__(256) k_boundary(DevBatch B) {
   if (overflowed(B)) return;
   constexpr int NV = MAX_NV;
@@ -1252,49 +1228,7 @@ __global__ void __launch_bounds__(256) k_boundary(DevBatch B) {
         es |= (uint32_t)B.segspin_new[top[a]] << a;
       }
     }
-    const uint32_t all = (1u << nv) - 1;
-    // words 0..3, and 4..7 when the two shuffles can take more than four
-    // (n_0 - 1 + n_1 - 1 <= nv - 1 words in all)
-    const U4 x0 = philox(B.sweep[c], STAGE_BOUNDARY, (uint32_t)r, 0u, P.key0, P.key1);
-    U4 x1 = {0u, 0u, 0u, 0u};
-    if (nv > 5) x1 = philox(B.sweep[c], STAGE_BOUNDARY, (uint32_t)r, 1u, P.key0, P.key1);
-    int k = 0;
-    uint32_t perm[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int n = __popc(u ? (bs & all) : (~bs & all));
-      uint32_t p = 0x76543210u;
-#pragma unroll
-      for (int i = NV - 1; i >= 1; --i) {
-        if (i < n) {
-          const uint32_t w = pick8(k, x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w);
-          const int j = i - (int)(w % (uint32_t)(i + 1));
-          ++k;
-          const uint32_t vi = (p >> (4 * i)) & 15u, vj = (p >> (4 * j)) & 15u;
-          p &= ~((15u << (4 * i)) | (15u << (4 * j)));
-          p |= (vi << (4 * j)) | (vj << (4 * i));
-        }
-      }
-      perm[u] = p;
-    }
-#pragma unroll
-    for (int a = 0; a < NV; ++a) {
-      if (a >= nv) continue;
-      const uint32_t u = (bs >> a) & 1u;
-      const uint32_t cls_b = u ? bs : ~bs, cls_e = u ? es : ~es;
-      const int rank = __popc(cls_b & all & ((1u << a) - 1));
-      const int t = (int)(((u ? perm[1] : perm[0]) >> (4 * rank)) & 15u);
-      // the top of spin u with rank t among the tops of spin u
-      int target = 0, cnt = 0;
-#pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        if (q < nv && ((cls_e >> q) & 1u)) {
-          if (cnt == t) target = q;
-          ++cnt;
-        }
-      }
-      uf_unite(B.parent, bot[a], pick8(target, top[0], top[1], top[2], top[3], top[4], top[5], top[6], top[7]));
-    }
+    join_boundary(P, B.sweep[c], r, bot, top, bs, es, [&](int a, int b) { uf_unite(B.parent, a, b); });
   }
 }
 
@@ -1370,12 +1304,6 @@ __device__ __forceinline__ int chunk_items(int M) {
 constexpr int HT_BITS = 10;
 constexpr int HT = 1 << HT_BITS;
 constexpr int HT_PROBES = 8;
-
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-  return v;
-}
 
 // Add one contribution (class lengths, tau = 0 boundary counts packed 8 bits
 // per class, packed winding) for root r to the block's LDS table, or to the
@@ -1654,48 +1582,6 @@ __global__ void __launch_bounds__(256) k_field_apply(DevBatch B) {
 constexpr int COL_THREADS = 256;
 constexpr int COL_MIN_CHUNK = 256 * 4;  // smallest collector chunk (256 * chunk_items)
 constexpr int COL_U = 4;                         // items per lane in flight (divides chunk_items)
-constexpr int NCOL = NUM_COLLECTOR_TERMS;
-
-// Collector terms of one cluster.  h, flip: the chain's field and the
-// cluster's flip; the field weight of the cluster is w = -h umag
-// (cluster.h:50-63) and its Zeeman energy after the flip flip ? -w : w
-// (path_integral.C:852-858).
-__device__ __forceinline__ void cluster_terms(const ClusterAcc& a, double h, int flip, double* v) {
-  const double L0 = a.L[0], L1 = a.L[1], L2 = a.L[2], L3 = a.L[3];
-  const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2], n3 = a.n[3];
-  int w0, w1;
-  unpack_winding(a.w, w0, w1);
-  // per-cluster improved estimates (susceptibility.h:96-147 with sigma = 1-2c)
-  const double usize0 = 0.5 * (n0 + n1 + n2 + n3), umag0 = 0.5 * (n0 + n1 - n2 - n3);
-  const double ssize0 = 0.5 * (n0 - n1 + n2 - n3), smag0 = 0.5 * (n0 - n1 - n2 + n3);
-  const double usize = 0.5 * ((L0 + L1) + (L2 + L3)), umag = 0.5 * ((L0 + L1) - (L2 + L3));
-  const double ssize = 0.5 * ((L0 - L1) + (L2 - L3)), smag = 0.5 * ((L0 - L1) - (L2 - L3));
-  v[0] = 1.0;  // clusters
-  v[1] = umag0;
-  v[2] = usize0 * usize0;
-  v[3] = umag0 * umag0;
-  v[4] = v[2] * v[2];
-  v[5] = v[3] * v[3];
-  v[6] = usize * usize;
-  v[7] = umag * umag;
-  v[8] = smag0;
-  v[9] = ssize0 * ssize0;
-  v[10] = smag0 * smag0;
-  v[11] = v[9] * v[9];
-  v[12] = v[10] * v[10];
-  v[13] = ssize * ssize;
-  v[14] = smag * smag;
-  v[15] = 0.25 * ((double)w0 * w0 + (double)w1 * w1);
-  v[16] = umag;   // normal estimator: tau-integrated magnetization
-  v[17] = smag;
-  const double wf = -h * umag;
-  v[18] = flip ? -wf : wf;
-}
-
-// record slot of collector term q (R_NC, R_UMAG0 .. R_W2, R_UMAGA, R_SMAGA, R_EFIELD)
-__device__ __forceinline__ int term_slot(int q) {
-  return q == 0 ? R_NC : (q <= 15 ? R_UMAG0 + (q - 1) : R_UMAGA + (q - 16));
-}
 
 // clear: zero each root's accumulator after reading it (no compress pass)
 __global__ void __launch_bounds__(COL_THREADS) k_flip_collect(DevBatch B, int clear) {
@@ -1937,8 +1823,8 @@ __global__ void __launch_bounds__(256) k_exchange(DevBatch B) {
     const int a = B.xslot[t], b = B.xslot[t + 1];
     const ChainDev& Pa = B.chains[a];
     const ChainDev& Pb = B.chains[b];
-    const int na = B.bo_new[Pa.bond_base + Pa.Nb] - B.bo_new[Pa.bond_base];
-    const int nb = B.bo_new[Pb.bond_base + Pb.Nb] - B.bo_new[Pb.bond_base];
+    const int na = B.blk_nops ? B.blk_nops[a] : B.bo_new[Pa.bond_base + Pa.Nb] - B.bo_new[Pa.bond_base];
+    const int nb = B.blk_nops ? B.blk_nops[b] : B.bo_new[Pb.bond_base + Pb.Nb] - B.bo_new[Pb.bond_base];
     const double x = (double)(na - nb) * B.xlnr[t];
     const bool accept = (x >= 0.0) || (log_uniform(philox(step, STAGE_EXCHANGE, (uint32_t)t, 0u, B.xkey0, B.xkey1)) < x);
     if (accept) {
@@ -2247,9 +2133,9 @@ int scan_blocks(const DevBatch& B) {
   return (B.nbonds + SCAN_CHUNK - 1) / SCAN_CHUNK + (B.nsites + SCAN_CHUNK - 1) / SCAN_CHUNK;
 }
 
-const char* const kKernelNames[NUM_SWEEP_KERNELS] = {
+const char* const kKernelNames[NUM_PROFILED] = {
     "diag_count", "scan", "diag_fill", "link",
-    "uf_union", "uf_compress", "estimate", "flip_collect", "end_sweep"};
+    "uf_union", "uf_compress", "estimate", "flip_collect", "end_sweep", "chain_sweep"};
 
 // ev (optional): NUM_SWEEP_KERNELS + 1 events recorded around the launches
 static inline void mark(hipEvent_t* ev, int i, hipStream_t st) {
@@ -2335,6 +2221,10 @@ void launch_cluster_stage(const DevBatch& B, const LaunchCfg& L, hipStream_t st,
   mark(ev, 5, st);
   hipLaunchKernelGGL(k_end_sweep, dim3(B.nchains), dim3(END_THREADS), 0, st, B);
   mark(ev, 6, st);
+  launch_exchange(B, st);
+}
+
+void launch_exchange(const DevBatch& B, hipStream_t st) {
   if (B.nslots > 1) hipLaunchKernelGGL(k_exchange, dim3(1), dim3(256), 0, st, B);
 }
 

@@ -237,6 +237,7 @@ def kernel_bytes(compress, link=0):
     if link == 0:
         b["link"] += b["uf_union"]
         b["uf_union"] = 0.0
+    b["chain_sweep"] = sum(BYTES_PER_OP.values())  # one workgroup per chain: the whole sweep
     return b
 
 
@@ -257,7 +258,8 @@ def roofline(prof, nop_mean, traffic_profile=None, compress=1, link=0):
 
 STAGES = {"diagonal update": ("diag_count", "scan", "diag_fill"),
           "linking": ("link",), "union-find": ("uf_union", "uf_compress"),
-          "estimators": ("estimate",), "flip + collect": ("flip_collect", "end_sweep")}
+          "estimators": ("estimate",), "flip + collect": ("flip_collect", "end_sweep"),
+          "one workgroup per chain": ("chain_sweep",)}
 
 
 def stage_gbs(prof, nop_mean, compress=1, link=0):

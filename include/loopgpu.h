@@ -215,7 +215,10 @@ int lg_exchange_state(lg_batch* h, int32_t* chain_at, uint64_t* accepted, uint64
  * estimator finds the roots itself; flush: the estimator flushes its LDS
  * cluster table to global memory every 256 * flush segments of its chunk
  * (4, 8 or 16).  By default they follow the expected operator counts, and
- * lg_batch_tune times the candidates.  set: fields < 0 keep their value; the settings then
+ * lg_batch_tune times the candidates.  Chains that fit one workgroup each are by
+ * default swept by one workgroup per chain, several sweeps per launch, when
+ * that is expected (or, by the tuner, measured) to be faster; these settings
+ * are the other kernels', which set selects.  set: fields < 0 keep their value; the settings then
  * stay as given (no automatic choice) until the next tune.  Results do not
  * depend on them.  No counterpart in the reference (launch configuration of
  * the device kernels). */
@@ -234,7 +237,8 @@ int lg_batch_set_launch(lg_batch* h, const lg_launch* l);
 /* ---- measurement ------------------------------------------------------------
  * n sweeps with HIP events recorded between the kernel launches on the
  * handle's stream; avg_ms[i] = mean duration per sweep of kernel i, in the
- * order of lg_profile_kernel_name(i), i < lg_profile_num_kernels().  The
+ * order of lg_profile_kernel_name(i), i < lg_profile_num_kernels() (where a
+ * workgroup sweeps each chain, all of the time is kernel "chain_sweep").  The
  * configuration advances by n sweeps (records are not returned).  These are
  * the reference's timer regions (path_integral.C:284-299) as device kernels. */
 int lg_profile_num_kernels(void);
