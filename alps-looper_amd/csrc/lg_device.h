@@ -15,6 +15,14 @@ __device__ __forceinline__ bool overflowed(const DevBatch& B) {
   return __hip_atomic_load(B.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
+// one thread, in the kernel before a scan: clear the ticket, next epoch
+// (never 0, the value of freshly cleared status words)
+__device__ __forceinline__ void scan_advance_epoch(const DevBatch& B) {
+  B.scan_ctl[0] = 0;
+  uint32_t e = ((uint32_t)B.scan_ctl[1] + 1u) & 0x3fffffffu;
+  B.scan_ctl[1] = (int)(e == 0 ? 1u : e);
+}
+
 __device__ __forceinline__ double wave_sum_d(double v) {
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);

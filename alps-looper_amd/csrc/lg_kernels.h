@@ -136,6 +136,11 @@ void launch_site_scan(const DevBatch& B, hipStream_t st);
 void launch_canon(const DevBatch& B, int chain, int nelem, int* canon, int* labels, int* roots,
                   hipStream_t st);
 int scan_blocks(const DevBatch& B);
+// the series walk of SSE chains, its string into bond-major operators, and
+// the flipped types back into the string (lg_sse.hip)
+void launch_sse_walk(const DevBatch& B, hipStream_t st);
+void launch_sse_scatter(const DevBatch& B, hipStream_t st);
+void launch_sse_gather(const DevBatch& B, hipStream_t st);
 // LDS that a workgroup of k_chain_sweeps can ask for (160 KB less its static part)
 constexpr int BLOCK_LDS_MAX = 160 * 1024 - 4096;
 int block_prepare();                          // 1 when the device grants that much

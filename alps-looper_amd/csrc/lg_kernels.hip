@@ -232,14 +232,6 @@ __device__ __forceinline__ unsigned long long scan_word(uint32_t epoch, int stat
   return ((unsigned long long)epoch << 34) | ((unsigned long long)state << 32) | (uint32_t)v;
 }
 
-// one thread, in the kernel before a scan: clear the ticket, next epoch
-// (never 0, the value of freshly cleared status words)
-__device__ __forceinline__ void scan_advance_epoch(const DevBatch& B) {
-  B.scan_ctl[0] = 0;
-  uint32_t e = ((uint32_t)B.scan_ctl[1] + 1u) & 0x3fffffffu;
-  B.scan_ctl[1] = (int)(e == 0 ? 1u : e);
-}
-
 // ---------------------------------------------------------------------------
 // (a) diagonal update, pass 1: count and store accepted candidates
 // ---------------------------------------------------------------------------
@@ -1880,219 +1872,6 @@ __global__ void k_canon_label(DevBatch B, int chain, int nelem, const int* canon
 }
 
 // ---------------------------------------------------------------------------
-// "loop; sse" (sse.C:174-400): the same loop clusters on the stochastic
-// series expansion.  A chain's operator string (series order) is walked by
-// one wave, all lanes carrying the same state: before each kept operator,
-// and again after each insertion, a gap tries an insertion when
-// (n + 1) u < beta W_tot (W_tot = Nb sum_g v_g; bond uniform from word 2,
-// graph from word 3 by the thresholds, kept if compatible); a diagonal
-// operator is removed when beta W_tot u < n (the next one follows with no gap
-// between) or else regraphed by choose_diagonal (graph_impl.h:297-312); an
-// off-diagonal one by choose_offdiagonal.  W_tot sums every location's
-// graphs: lattice bonds, the single-ion term's in-site bonds and the
-// transverse field's site operators (the site graph, always compatible; an
-// off-diagonal site operator flips its one spin).  Step k of the walk takes the words
-// Philox(sweep, 6, 0, k), computed 64 steps at a time, one per lane, and
-// staged in LDS with the spins, the per-bond counters and sites and the
-// operators in flight, so that a step waits on no global memory.  The new string then becomes bond-major operators at times p / n, on
-// which the path-integral cluster stage runs unchanged (lengths in units of
-// the string), and the flipped types return to the string.
-// ---------------------------------------------------------------------------
-constexpr int SSE_THREADS = 64;
-
-__global__ void __launch_bounds__(SSE_THREADS) k_sse_diag(DevBatch B) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) scan_advance_epoch(B);  // for k_scan, which follows
-  if (overflowed(B)) return;
-  const int c = blockIdx.x;
-  // (a copy: the string stores below could alias the descriptor, which
-  // would make every step reload its fields)
-  const ChainDev P = B.chains[c];
-  // The walk's working set in LDS, so that a step waits on no global memory:
-  // spins, per-bond counters, each bond's two sites, the next 64 old
-  // operators and the last (up to 64) emitted ones, stored 64 at a time
-  __shared__ uint8_t spc[SSE_MAX_SITES];
-  __shared__ int cnt[SSE_MAX_BONDS];
-  __shared__ uint32_t ends[SSE_MAX_BONDS];  // source | target << 16
-  __shared__ int ochunk[SSE_THREADS], obuf[SSE_THREADS];
-  __shared__ U4 xbuf[SSE_THREADS];          // the Philox words of the next 64 steps
-  const int lane = threadIdx.x;
-  const int Nb = P.Nb;
-  for (int s = lane; s < P.N; s += SSE_THREADS) spc[s] = B.spins_old[P.old_site_base + s];
-  for (int b = lane; b < Nb; b += SSE_THREADS) {
-    int s0, s1;
-    op_sites(P, b, s0, s1);
-    cnt[b] = 0;
-    ends[b] = (uint32_t)s0 | ((uint32_t)s1 << 16);
-  }
-  __syncthreads();
-  const uint32_t sweep = B.sweep[c];
-  const int n_old = B.bo_old[P.old_bond_base + Nb] - B.bo_old[P.old_bond_base];
-  const int* so = B.sse_old + P.sse_base;
-  int* sn = B.sse_new + P.sse_base;
-  const double bw = P.beta * P.sse_wtot;
-  int nop = n_old, out = 0, i = 0, step = 0;
-  int xbase = -SSE_THREADS, obase = -SSE_THREADS;  // first step / old operator held by the lanes
-  bool try_gap = true, full = false;
-  // Every lane runs the walk on the same values; reading each value loaded
-  // from LDS through readfirstlane tells the compiler so, which keeps the
-  // walk's state in scalar registers and its branches scalar.
-  auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-  while (try_gap || i < n_old) {
-    if (step - xbase >= SSE_THREADS) {
-      xbase = step;
-      xbuf[lane] = philox(sweep, STAGE_SSE, 0u, (uint32_t)(step + lane), P.key0, P.key1);
-    }
-    U4 x = xbuf[step - xbase];  // (one wave: its LDS accesses complete in order)
-    x.x = (uint32_t)uni((int)x.x);
-    x.y = (uint32_t)uni((int)x.y);
-    x.z = (uint32_t)uni((int)x.z);
-    x.w = (uint32_t)uni((int)x.w);
-    ++step;
-    const double u = uniform53(x);
-    int ne, b;
-    if (try_gap) {
-      try_gap = false;
-      if (!((double)(nop + 1) * u < bw)) continue;
-      // the location's class and graph by word 2, the location by word 3
-      // (the thresholds ascend, so g counts those at or below z; no array
-      // of the descriptor is indexed at run time, which would put the
-      // whole copy in scratch memory)
-      const uint64_t z = x.z;
-      int g = 0;
-      if (z < P.sse_cls[0]) {
-        b = (int)(((uint64_t)x.w * (uint64_t)P.nb_lat) >> 32);
-        g = (int)(z >= P.sse_tl[0]) + (int)(z >= P.sse_tl[1]) + (int)(z >= P.sse_tl[2]);
-      } else if (z < P.sse_cls[1]) {
-        b = P.nb_lat + (int)(((uint64_t)x.w * (uint64_t)(P.nb_real - P.nb_lat)) >> 32);
-        g = (int)(z >= P.sse_td[0]) + (int)(z >= P.sse_td[1]) + (int)(z >= P.sse_td[2]);
-      } else {  // a site operator: the site graph, compatible with either spin
-        b = P.nb_real + (int)(((uint64_t)x.w * (uint64_t)P.N) >> 32);
-      }
-      if (b < P.nb_real) {
-        const uint32_t e2 = (uint32_t)uni((int)ends[b]);
-        if (((g & 1) ^ uni(spc[e2 & 0xffff]) ^ uni(spc[e2 >> 16])) == 0) continue;
-      }
-      ne = (b << 3) | (g << 1);
-      ++nop;
-    } else {
-      if (i - obase >= SSE_THREADS) {  // the next 64 old operators
-        obase = i;
-        ochunk[lane] = (i + lane < n_old) ? so[i + lane] : 0;
-      }
-      const int e = uni(ochunk[i - obase]);
-      ++i;
-      b = e >> 3;
-      const uint32_t e2 = (uint32_t)uni((int)ends[b]);
-      const int s0 = (int)(e2 & 0xffff), s1 = (int)(e2 >> 16);
-      const int c0 = uni(spc[s0]), c1 = uni(spc[s1]);
-      const bool site = b >= P.nb_real, insite = b >= P.nb_lat && !site;
-      if ((e & 1) == 0) {
-        if (bw * u < (double)nop) {  // removed
-          --nop;
-          continue;
-        }
-        const int cc = 1 ^ c0 ^ c1;  // 0 antiparallel, 1 parallel
-        const uint64_t pd = insite ? (cc ? P.dpdiag[1] : P.dpdiag[0]) : (cc ? P.pdiag[1] : P.pdiag[0]);
-        ne = (b << 3) | (site ? 0 : (((((uint64_t)x.z < pd) ? 0 : 2) ^ cc) << 1));
-      } else {
-        const uint64_t to = insite ? P.dtoff : P.toff;
-        ne = (b << 3) | (site ? 0 : ((((uint64_t)x.z < to) ? 0 : 1) << 1)) | 1;
-        if (lane == 0) {
-          spc[s0] = (uint8_t)(c0 ^ 1);
-          if (!site) spc[s1] = (uint8_t)(c1 ^ 1);  // a site operator flips its one spin
-        }
-      }
-    }
-    if (out >= P.sse_cap) {
-      full = true;
-      break;
-    }
-    if (lane == 0) {
-      obuf[out & (SSE_THREADS - 1)] = ne;
-      atomicAdd(&cnt[b], 1);
-    }
-    ++out;
-    if ((out & (SSE_THREADS - 1)) == 0) sn[out - SSE_THREADS + lane] = obuf[lane];  // 64 emitted
-    try_gap = true;
-  }
-  const int rest = out & (SSE_THREADS - 1);
-  if (lane < rest) sn[out - rest + lane] = obuf[lane];
-  if (full && lane == 0) atomicOr(B.flags, FLAG_OP_OVERFLOW);
-  __syncthreads();
-  for (int b = lane; b < Nb; b += SSE_THREADS) B.counts[P.bond_base + b] = cnt[b];
-}
-
-// the new string into bond-major order (series order within a bond), times
-// p / n; perm[p] = the operator index of string position p
-__global__ void __launch_bounds__(SSE_THREADS) k_sse_scatter(DevBatch B) {
-  if (overflowed(B)) return;
-  const int c = blockIdx.x;
-  const ChainDev P = B.chains[c];  // (a copy, as in k_sse_diag)
-  __shared__ int cur[SSE_MAX_BONDS], koff[SSE_MAX_BONDS];
-  const int lane = threadIdx.x, Nb = P.Nb;
-  for (int b = lane; b < Nb; b += SSE_THREADS) {
-    cur[b] = B.bo_new[P.bond_base + b];
-    koff[b] = 0;
-  }
-  __syncthreads();
-  const int n = B.bo_new[P.bond_base + Nb] - B.bo_new[P.bond_base];
-  const int* sn = B.sse_new + P.sse_base;
-  int* perm = B.sse_perm + P.sse_base;
-  const double dn = (double)n;
-  for (int p0 = 0; p0 < n; p0 += SSE_THREADS) {
-    // lanes past the end hold -1 (bond -1, which no element has)
-    const int el = (p0 + lane < n) ? sn[p0 + lane] : -1;
-    const int m = min(SSE_THREADS, n - p0);
-    // in series order, each element takes its bond's next slot and
-    // off-diagonal count: the elements of the same bond before it in these
-    // 64 add to the bond's counts so far, and the last of them carries the
-    // counts on to the next 64
-    int rank = 0, roff = 0;
-    bool last = true;
-    for (int j = 0; j < m; ++j) {
-      const int e = __shfl(el, j);
-      if ((e >> 3) == (el >> 3)) {
-        if (j < lane) {
-          ++rank;
-          roff += e & 1;
-        } else if (j > lane) {
-          last = false;
-        }
-      }
-    }
-    if (p0 + lane < n) {
-      const int b = el >> 3;
-      const int pos = cur[b] + rank, kc = koff[b] + roff;
-      if (last) {  // (one wave: these stores follow every lane's loads above)
-        cur[b] = pos + 1;
-        koff[b] = kc + (el & 1);
-      }
-      B.ot_new[pos] = (double)(p0 + lane) / dn;
-      B.oi_new[pos] = ((P.bond_base + b) << 3) | (el & 7);
-      B.kc_new[pos] = kc;
-      perm[p0 + lane] = pos;
-    }
-  }
-  // each bond's diagonal operators, as the path-integral diagonal update
-  // leaves them (k_end_sweep counts the off-diagonal ones for the sign)
-  __syncthreads();
-  for (int b = lane; b < Nb; b += SSE_THREADS)
-    B.acc_count[P.bond_base + b] = (cur[b] - B.bo_new[P.bond_base + b]) - koff[b];
-}
-
-// the flipped operator types back into the string
-__global__ void __launch_bounds__(256) k_sse_gather(DevBatch B) {
-  if (overflowed(B)) return;
-  const int c = blockIdx.x;
-  const ChainDev& P = B.chains[c];
-  // (k_end_sweep has moved the chain's old bases to the configuration just built)
-  const int o0 = B.bo_new[P.bond_base], n = B.bo_new[P.bond_base + P.Nb] - o0;
-  int* sn = B.sse_new + P.sse_base;
-  const int* perm = B.sse_perm + P.sse_base;
-  for (int p = threadIdx.x; p < n; p += blockDim.x) sn[p] = (sn[p] & ~1) | (B.oi_new[perm[p]] & 1);
-}
-
-// ---------------------------------------------------------------------------
 // host-side launchers
 // ---------------------------------------------------------------------------
 template <int G>
@@ -2144,14 +1923,14 @@ static inline void mark(hipEvent_t* ev, int i, hipStream_t st) {
 
 static void launch_sweep_sse(const DevBatch& B, const LaunchCfg& L, hipStream_t st, hipEvent_t* ev) {
   mark(ev, 0, st);
-  hipLaunchKernelGGL(k_sse_diag, dim3(B.nchains), dim3(SSE_THREADS), 0, st, B);  // also the scan's epoch
+  launch_sse_walk(B, st);  // also the scan's epoch
   mark(ev, 1, st);
   hipLaunchKernelGGL(k_scan, dim3(scan_blocks(B)), dim3(SCAN_THREADS), 0, st, B);
   mark(ev, 2, st);
-  hipLaunchKernelGGL(k_sse_scatter, dim3(B.nchains), dim3(SSE_THREADS), 0, st, B);
+  launch_sse_scatter(B, st);
   mark(ev, 3, st);
   launch_cluster_stage(B, L, st, ev ? ev + 3 : nullptr);
-  hipLaunchKernelGGL(k_sse_gather, dim3(B.nchains), dim3(256), 0, st, B);
+  launch_sse_gather(B, st);
 }
 
 void launch_sweep(const DevBatch& B, const LaunchCfg& L, hipStream_t st, hipEvent_t* ev) {
