@@ -269,6 +269,7 @@ void Batch::release() {
   for (void* p : allocations) hipFree(p);
   allocations.clear();
   if (rec_host) { hipHostFree(rec_host); rec_host = nullptr; }
+  if (cfg_host) { hipHostFree(cfg_host); cfg_host = nullptr; }
   if (stream) { hipStreamDestroy(stream); stream = nullptr; }
 }
 
@@ -513,16 +514,21 @@ int Batch::allocate(bool dynamic) {
   blk_lds_grant = !dynamic && block_prepare() ? BLOCK_LDS_MAX : 0;
   if ((rc = alloc(col_part, (size_t)col_chunks(node_cap) * NUM_COLLECTOR_TERMS))) return rc;
   if ((rc = alloc(totals, 2))) return rc;
-  if ((rc = alloc(flags, 1))) return rc;
   if ((rc = alloc(d_sweep, cap_chains))) return rc;
   if ((rc = alloc(rec_acc, (size_t)cap_chains * R_COUNT))) return rc;
   ring_size = (int)std::max<long long>(16, std::min<long long>(4096, (64ll << 20) / ((long long)cap_chains * R_COUNT * 8)));
-  if ((rc = alloc(rec_ring, (size_t)ring_size * cap_chains * R_COUNT))) return rc;
+  // the error flags stand before the record ring, so that one copy brings both
+  // to the host
+  const size_t rec_words = REC_HEAD + (size_t)ring_size * cap_chains * R_COUNT;
+  double* rec_block = nullptr;
+  if ((rc = alloc(rec_block, rec_words))) return rc;
+  flags = (int*)rec_block;
+  rec_ring = rec_block + REC_HEAD;
   // records reach the host through pinned memory: a copy to pageable memory
   // of a size not seen before costs the runtime milliseconds of staging
   if (rec_host) { hipHostFree(rec_host); rec_host = nullptr; }
   {
-    const hipError_t e = hipHostMalloc((void**)&rec_host, (size_t)ring_size * cap_chains * R_COUNT * sizeof(double));
+    const hipError_t e = hipHostMalloc((void**)&rec_host, rec_words * sizeof(double));
     if (e != hipSuccess) {
       rec_host = nullptr;
       return set_error(LG_ERR_DEVICE, std::string("hipHostMalloc of the record mirror: ") + hipGetErrorString(e));
@@ -532,7 +538,9 @@ int Batch::allocate(bool dynamic) {
   if ((rc = alloc(end_count, 1))) return rc;
   LG_HIP(hipMemset(end_count, 0, sizeof(int)));
   LG_HIP(hipMemset(rec_acc, 0, (size_t)cap_chains * R_COUNT * sizeof(double)));
-  LG_HIP(hipMemset(flags, 0, sizeof(int)));
+  LG_HIP(hipMemset(flags, 0, REC_HEAD * sizeof(double)));
+  flags_seen = 0;
+  known_ops.clear();
   LG_HIP(hipMemset(ring_pos, 0, sizeof(int)));
   LG_HIP(hipMemset(totals, 0, 2 * sizeof(int)));
   int dev = 0;
@@ -811,6 +819,7 @@ int Batch::apply_cfg(const LaunchCfg& c) {
 
 // all-up spins, empty operator string (path_integral.C:225) for every chain
 int Batch::reset_state() {
+  known_ops.clear();
   cur = 0;
   blk_regions = false;
   State& s = st[cur];
@@ -840,6 +849,7 @@ int Batch::reset_state() {
 // after its current extent.  Nothing is copied on the device; the next sweep
 // reads each chain at its old bases and writes the new layout.
 int Batch::relayout(const std::vector<int>& keep, const std::vector<lg_params>& add) {
+  known_ops.clear();
   if (is_sse()) return set_error(LG_ERR_UNSUPPORTED, "relayout of SSE chains is not built");
   for (const auto& p : add)
     if (p.algorithm != LG_ALGORITHM_PATH_INTEGRAL) return set_error(LG_ERR_UNSUPPORTED, "SSE chains are not served");
@@ -962,9 +972,9 @@ int Batch::capture(int from) {
   return LG_OK;
 }
 
-int Batch::check_flags() {
-  int f = 0;
-  LG_HIP(hipMemcpy(&f, flags, sizeof(int), hipMemcpyDeviceToHost));
+// the device's error flags as the host last saw them
+int Batch::flags_error() const {
+  const int f = flags_seen;
   if (f) {
     std::string m = "device capacity exceeded:";
     if (f & FLAG_CAND_OVERFLOW) m += " candidate slots";
@@ -974,6 +984,11 @@ int Batch::check_flags() {
     return set_error(LG_ERR_CAPACITY, m);
   }
   return LG_OK;
+}
+
+int Batch::check_flags() {
+  LG_HIP(hipMemcpy(&flags_seen, flags, sizeof(int), hipMemcpyDeviceToHost));
+  return flags_error();
 }
 
 int Batch::enqueue_sweep() {
@@ -1001,10 +1016,11 @@ void Batch::note_swept() {
 }
 
 int Batch::run(uint32_t n, lg_sweep_record* out) {
-  int rc = check_flags();
+  int rc = flags_error();  // (every call that sweeps leaves the flags it ended with)
   if (rc) return rc;
   const size_t nc = chains.size();
-  if (nc == 0) return LG_OK;
+  if (nc == 0 || n == 0) return LG_OK;
+  known_ops.clear();
   const bool block = block_form();
   if (!block && (rc = ensure_packed())) return rc;
   uint32_t done = 0;
@@ -1019,14 +1035,18 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
         if (rc) return rc;
       }
     }
-    const size_t words = (size_t)chunk * nc * R_COUNT;
-    if (out) LG_HIP(hipMemcpyAsync(rec_host, rec_ring, words * sizeof(double), hipMemcpyDeviceToHost, stream));
+    // one copy for the flags and the records
+    const size_t words = out ? (size_t)chunk * nc * R_COUNT : 0;
+    LG_HIP(hipMemcpyAsync(rec_host, flags, (REC_HEAD + words) * sizeof(double), hipMemcpyDeviceToHost, stream));
     LG_HIP(hipStreamSynchronize(stream));
-    rc = check_flags();
-    if (rc) return rc;
+    std::memcpy(&flags_seen, rec_host, sizeof(int));
+    if ((rc = flags_error())) return rc;
     if (out) {
       static_assert(sizeof(lg_sweep_record) == R_COUNT * sizeof(double), "record layout");
-      std::memcpy(out + (size_t)done * nc, rec_host, words * sizeof(double));
+      std::memcpy(out + (size_t)done * nc, rec_host + REC_HEAD, words * sizeof(double));
+      if (done + chunk == n)  // the configurations' operator counts
+        for (size_t c = 0; c < nc; ++c)
+          known_ops.push_back((long long)rec_host[REC_HEAD + ((size_t)(chunk - 1) * nc + c) * R_COUNT + R_NOP]);
     }
     for (size_t c = 0; c < nc; ++c) host_sweep[c] += chunk;
     done += chunk;
@@ -1141,6 +1161,7 @@ int Batch::profile(uint32_t n, double* ms) {
   if (rc) return rc;
   const int K = NUM_SWEEP_KERNELS;
   for (int i = 0; i < NUM_PROFILED; ++i) ms[i] = 0;
+  known_ops.clear();
   if (block_form()) {  // one workgroup per chain: the launches as a whole
     hipEvent_t e0, e1;
     LG_HIP(hipEventCreate(&e0));
@@ -1268,6 +1289,7 @@ int Batch::set_config(int c, const int32_t* spins_in, const int32_t* bond_offset
   int rc = validate_config(d, bond_offsets, times, types, nops);
   if (rc) return rc;
   if (nops > op_cap) return set_error(LG_ERR_CAPACITY, "configuration exceeds operator capacity");
+  known_ops.clear();
   std::vector<int> spins(spins_in, spins_in + d.N), bo(bond_offsets, bond_offsets + d.Nb + 1), offd(nops);
   std::vector<double> ot(times, times + nops);
   std::vector<int> oi(nops);
@@ -1315,10 +1337,52 @@ int Batch::set_config(int c, const int32_t* spins_in, const int32_t* bond_offset
   return sync_schedule();
 }
 
+// A chain's configuration in the ABI's layout, written straight to the host's
+// (mapped) memory: four blocking copies took 40 us for a 16-site chain.
+__global__ void __launch_bounds__(256) k_export(const uint8_t* spins, const int* bo, const double* ot, const int* oi,
+                                                int N, int Nb, int nops, int32_t* out_spins, int32_t* out_bo,
+                                                double* out_times, int32_t* out_types) {
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  const int op0 = bo[0];
+  if (out_spins)
+    for (int s = t0; s < N; s += stride) out_spins[s] = spins[s];
+  if (out_bo)
+    for (int b = t0; b <= Nb; b += stride) out_bo[b] = bo[b] - op0;
+  if (out_times)
+    for (int k = t0; k < nops; k += stride) out_times[k] = ot[op0 + k];
+  if (out_types)
+    for (int k = t0; k < nops; k += stride) {
+      const int v = oi[op0 + k];
+      out_types[k] = (v & 1) | (((v >> 1) & 3) << 2);
+    }
+}
+
 int Batch::get_config(int c, int32_t* spins, int32_t* bond_offsets, double* times, int32_t* types) {
   if (chains.size() != 1) return set_error(LG_ERR_UNSUPPORTED, "get_config needs a single-chain handle");
   const ChainDev& d = chains[c];
   const State& s = st[cur];
+  const bool ops = times || types;
+  if (!ops || !known_ops.empty()) {
+    const size_t n = ops ? (size_t)known_ops[c] : 0;
+    const size_t bytes = n * 12 + ((size_t)d.N + d.Nb + 1) * 4;
+    if (bytes <= CFG_HOST_BYTES && !cfg_host && hipHostMalloc((void**)&cfg_host, CFG_HOST_BYTES) != hipSuccess) cfg_host = nullptr;
+    if (bytes <= CFG_HOST_BYTES && cfg_host) {
+      double* const ht = (double*)cfg_host;
+      int32_t* const hy = (int32_t*)(ht + n);
+      int32_t* const hs = hy + n;
+      int32_t* const hb = hs + d.N;
+      const int blocks = (int)std::min<size_t>(64, (n + d.N + d.Nb + 256) / 256);
+      hipLaunchKernelGGL(k_export, dim3(blocks), dim3(256), 0, stream, s.spins, s.bo, s.ot, s.oi, d.N, d.Nb, (int)n,
+                         spins ? hs : nullptr, bond_offsets ? hb : nullptr, times ? ht : nullptr, types ? hy : nullptr);
+      LG_HIP(hipGetLastError());
+      LG_HIP(hipStreamSynchronize(stream));
+      if (spins) std::memcpy(spins, hs, (size_t)d.N * 4);
+      if (bond_offsets) std::memcpy(bond_offsets, hb, ((size_t)d.Nb + 1) * 4);
+      if (times) std::memcpy(times, ht, n * 8);
+      if (types) std::memcpy(types, hy, n * 4);
+      return LG_OK;
+    }
+  }
   std::vector<uint8_t> sp(d.N);
   std::vector<int> bo(d.Nb + 1);
   LG_HIP(hipMemcpy(sp.data(), s.spins, d.N, hipMemcpyDeviceToHost));
@@ -1336,6 +1400,10 @@ int Batch::get_config(int c, int32_t* spins, int32_t* bond_offsets, double* time
 }
 
 int Batch::num_ops(int c, long long* n) {
+  if ((size_t)c < known_ops.size()) {
+    *n = known_ops[c];
+    return LG_OK;
+  }
   if (blk_regions) {
     int v = 0;
     LG_HIP(hipMemcpy(&v, blk_nops + c, sizeof(int), hipMemcpyDeviceToHost));
@@ -1381,6 +1449,7 @@ int Batch::chain_config(int c, std::vector<int>& spins, std::vector<int>& bo, st
 int Batch::load_configs(const std::vector<HostConfig>& cfg) {
   if (cfg.size() != chains.size()) return set_error(LG_ERR_ARG, "one configuration per chain");
   blk_regions = false;
+  known_ops.clear();
   std::vector<uint8_t> sp(std::max(nsites, 1));
   std::vector<int> bo(nbonds + 1), soff(nsites + 1);
   std::vector<double> ot, evt;
@@ -1472,6 +1541,7 @@ void Batch::adopt(Batch& o) {
   const double capture_s = graph_capture_s;
   *this = o;  // member-wise: device pointers, host tables, settings
   o.rec_host = nullptr;
+  o.cfg_host = nullptr;
   graph_captures += captures;  // the counters cover the handle's lifetime
   graph_capture_s += capture_s;
   o.allocations.clear();

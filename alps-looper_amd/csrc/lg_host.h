@@ -149,6 +149,7 @@ class Batch {
   int apply_cfg(const LaunchCfg& c);
   int capture(int from);
   int check_flags();
+  int flags_error() const;
   void choose_block();
   int run_block(uint32_t n, uint32_t slot0);
   // st[cur] in the packed form (the chains' operators and segments consecutive)
@@ -188,7 +189,12 @@ class Batch {
   uint32_t* d_sweep = nullptr;
   double* rec_acc = nullptr;
   double* rec_ring = nullptr;
-  double* rec_host = nullptr;     // pinned host mirror of the record ring (hipHostMalloc)
+  double* rec_host = nullptr;     // pinned host mirror of the flags and the record ring (hipHostMalloc)
+  static constexpr size_t REC_HEAD = 8;           // words before the ring: the flags
+  unsigned char* cfg_host = nullptr;              // pinned memory for a configuration on its way out
+  static constexpr size_t CFG_HOST_BYTES = 256 << 10;
+  int flags_seen = 0;                             // the error flags as last read
+  std::vector<long long> known_ops;               // operators per chain, while the last records tell them
   int* ring_pos = nullptr;
   int* end_count = nullptr;
   int ring_size = 0;

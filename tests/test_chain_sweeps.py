@@ -60,3 +60,26 @@ def test_batches_cold_chains_and_changes_of_form(loopgpu):
     a.set_launch(group=16)
     print("flat", flush=True)
     _same(a.run(2), b.run(2))
+
+
+@pytest.mark.parametrize("kind,L,beta", [(0, 16, 4.0), (1, 32, 6.0), (1, 48, 12.0)])  # below and above the export's 256 KB
+def test_configuration_by_either_way_out(loopgpu, kind, L, beta):
+    """operator counts known from the last records, or asked from the device;
+    spins alone; after a configuration was set"""
+    c = loopgpu.Chain(loopgpu.params(kind, L, beta, seed=3))
+    print("config", kind, L, beta, flush=True)
+    c.sweep(7)
+    a = c.get_config()
+    spins = np.zeros(c.n_sites, np.int32)
+    assert loopgpu.lib.lg_chain_get_config(c.h, spins.ctypes.data, None, None, None) == 0
+    assert np.array_equal(spins, a[0])
+    d = loopgpu.Chain(loopgpu.params(kind, L, beta, seed=3))
+    d.sweep(7, records=False)
+    for x, y in zip(a, d.get_config()):
+        assert np.array_equal(x, y)
+    d.sweep(3)
+    d.set_config(*a, 7)
+    assert d.info() == c.info()
+    for x, y in zip(a, d.get_config()):
+        assert np.array_equal(x, y)
+    assert np.array_equal(c.sweep(2)[:, :2], d.sweep(2)[:, :2])
