@@ -266,6 +266,10 @@ __device__ __forceinline__ void blk_unite(const U& u, int a, int b) {
   }
 }
 
+// A segment's flags here (bits 0-1: its class, as ClusterAcc counts it; bits
+// 2-3: the winding of the event above it, for the event's source site)
+enum : uint8_t { SEG_GAUGE = 1, SEG_DOWN = 2, SEG_X = 4, SEG_Y = 8, SEG_FIRST = 16, SEG_EMPTY = 32, SEG_NOWRAP = 64 };
+
 // ---------------------------------------------------------------------------
 // a chain's working state, the same in every thread of its workgroup
 // ---------------------------------------------------------------------------
@@ -443,7 +447,7 @@ __device__ __forceinline__ void blk_link(const ChainDev& P, const Chain& S, cons
     const uint32_t e = S.ends[b];
     const bool site = GEN && b >= P.nb_real;
     const bool lattice = !GEN || b < P.nb_lat;
-    const uint8_t dflag = GEN ? (uint8_t)((lattice && bond_dir(P, b)) ? EV_DIR1 : 0) : (uint8_t)((chain || (b & 1)) ? 0 : EV_DIR1);
+    const int dflag = GEN ? (!lattice ? 0 : (bond_dir(P, b) ? SEG_Y : SEG_X)) : ((chain || (b & 1)) ? SEG_X : SEG_Y);
     const int own = k - S.bn[b], kpar = par(k);
     int leg[2];
 #pragma unroll
@@ -500,13 +504,13 @@ __device__ __forceinline__ void blk_link(const ChainDev& P, const Chain& S, cons
       }
       const int node = S.sn[s] + rank;
       const bool split = GEN && P.nv > 1;
-      const uint8_t gflag = (base & 2) ? EV_GAUGE : 0;
+      const int gflag = (base >> 1) & SEG_GAUGE;
       evt[node] = tau;
-      evflags[node] = (uint8_t)((info & 1) | ((side || !lattice) ? 0 : EV_SRC) | dflag | (rank == 0 ? EV_FIRST : 0) |
-                                gflag | (split && rank == 0 ? EV_NOWRAP : 0) | ((sp & 1) << 7));
+      evflags[node] = (uint8_t)(gflag | ((sp & 1) << 1) | (side ? 0 : dflag) | (rank == 0 ? SEG_FIRST : 0) |
+                                (split && rank == 0 ? SEG_NOWRAP : 0));
       if (split && node + 2 == S.sn[s + 1]) {  // the last event: the site's top segment, up to tau = 1
         evt[node + 1] = 1.0;
-        evflags[node + 1] = (uint8_t)(gflag | (((sp ^ info) & 1) << 7));
+        evflags[node + 1] = (uint8_t)(gflag | (((sp ^ info) & 1) << 1));
       }
       leg[side] = node;
     }
@@ -568,8 +572,8 @@ __device__ __forceinline__ int blk_clusters(const ChainDev& P, const Chain& S, c
         if (a < P.nv) {
           bot[a] = S.sn[r * P.nv + a];
           top[a] = S.sn[r * P.nv + a + 1] - 1;
-          bs |= (uint32_t)(evflags[bot[a]] >> 7) << a;
-          es |= (uint32_t)(evflags[top[a]] >> 7) << a;
+          bs |= (uint32_t)((evflags[bot[a]] >> 1) & 1) << a;
+          es |= (uint32_t)((evflags[top[a]] >> 1) & 1) << a;
         }
       }
       join_boundary(P, sweep, r, bot, top, bs, es, [&](int a, int b) { blk_unite(u, a, b); });
@@ -597,16 +601,22 @@ __device__ __forceinline__ int blk_clusters(const ChainDev& P, const Chain& S, c
 // segments of the 4 classes (16 bits each), the packed winding
 constexpr int ACC_BYTES = 48;
 struct Acc {
-  double* L;              // [4][W]
+  double* L;              // [W][4]
   unsigned long long* n;  // [W]
   unsigned long long* w;  // [W]
   int W;
-  __device__ __forceinline__ void add(int a, double len, int cls, bool first, int dw0, int dw1) const {
-    unsafeAtomicAdd(&L[cls * W + a], len);
-    if (first) atomicAdd(&n[a], 1ull << (16 * cls));
-    if (dw0 | dw1) atomicAdd(&w[a], (unsigned long long)pack_winding(dw0, dw1));
+  // a segment of cluster a: its length, and the winding d0, d1 (-1 .. 1)
+  __device__ __forceinline__ void add(int a, double len, int cls, int d0, int d1) const {
+    unsafeAtomicAdd(&L[4 * a + cls], len);
+    if (d0 | d1) atomicAdd(&w[a], (unsigned long long)pack_winding(d0, d1));
   }
 };
+// winding of a segment with flags fl above one with flags flo (stiffness.h:94-105)
+__device__ __forceinline__ void seg_winding(int fl, int flo, int& d0, int& d1) {
+  const int x = ((fl >> 2) & 1) - ((flo >> 2) & 1), y = ((fl >> 3) & 1) - ((flo >> 3) & 1);
+  d0 = (fl & SEG_DOWN) ? -x : x;
+  d1 = (fl & SEG_DOWN) ? -y : y;
+}
 
 }  // namespace
 
@@ -688,7 +698,6 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
   int* const l0 = B.l0 + P.blk_op;
   int* const l1 = B.l1 + P.blk_op;
   uint8_t* const evflags = B.evflags + P.blk_node;
-  int* const node_site = B.node_site + P.blk_node;
   int* const parents = B.parent + P.blk_node;
   int* const root_of = A.root_of + P.blk_node;
   double* const seg_len = A.seg_len + P.blk_node;
@@ -771,11 +780,9 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
     }
     for (int s = tid; s < N; s += T) {
       const int node = S.sn[s];
-      node_site[node] = s;
       if (S.sbase[s] & 1) {  // event-free site: one segment spanning [0,1)
         evt_new[node] = EMPTY_TIME;
-        evflags[node] = (uint8_t)(EV_EMPTY | EV_FIRST | ((S.sbase[s] & 2) ? EV_GAUGE : 0) |
-                                  (GEN && P.nv > 1 ? EV_NOWRAP : 0) | (S.spin[s] << 7));
+        evflags[node] = (uint8_t)(SEG_EMPTY | SEG_FIRST | ((S.sbase[s] >> 1) & SEG_GAUGE) | (S.spin[s] << 1));
       }
     }
     // ---- the new operator list ----
@@ -901,47 +908,34 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
     if (direct)
       for (int i = tid; i < 6 * ac.W; i += T) ((unsigned long long*)wbase)[i] = 0;
     __syncthreads();
+    auto root_at = [&](int x) -> int { return lds_p ? (int)p16[x] : ParentsMem{parents}.get(x); };
+    // a segment's terms: into its cluster's accumulator, or to memory
+    auto account = [&](int x, int id, double len, int fl, int flo) {
+      int d0, d1;
+      seg_winding(fl, flo, d0, d1);
+      if (direct) {
+        ac.add(id, len, fl & 3, d0, d1);
+      } else {
+        seg_len[x] = len;
+        seg_info[x] = (uint32_t)id | ((uint32_t)(fl & 3) << 24) | ((uint32_t)(fl & SEG_FIRST) << 22) |
+                      ((uint32_t)(d0 + 1) << 27) | ((uint32_t)(d1 + 1) << 29);
+      }
+    };
     {
       // U segments per thread at a time, every load of them before its use
-      constexpr int U = 4;
+      constexpr int U = 2;
       const int end = mw * 64;
       for (int x0 = tid; x0 < end; x0 += U * T) {
-        int xc[U], root[U], id[U];
-        uint8_t fl[U], flo[U];
+        int root[U], fl[U], flo[U];
         double thi[U], tlo[U];
-        bool anyfirst = false;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          xc[u] = min(x0 + u * T, m - 1);
-          fl[u] = evflags[xc[u]];
-          thi[u] = evt_new[xc[u]];
-          const int lower = max(xc[u] - 1, 0);  // replaced below for a site's first segment
+          const int x = min(x0 + u * T, m - 1), lower = max(x - 1, 0);
+          fl[u] = evflags[x];
+          thi[u] = evt_new[x];
           tlo[u] = evt_new[lower];
           flo[u] = evflags[lower];
-          root[u] = lds_p ? (int)p16[xc[u]] : ParentsMem{parents}.get(xc[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          id[u] = roots.rank(root[u]);
-          anyfirst |= (fl[u] & EV_FIRST) != 0;
-        }
-        if (__ballot(anyfirst)) {
-          // the segment below a site's first one is its last (the site's line
-          // wraps through tau = 1); a virtual site's starts at tau = 0
-          int last[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) last[u] = node_site[(fl[u] & EV_FIRST) ? xc[u] : 0];
-#pragma unroll
-          for (int u = 0; u < U; ++u) last[u] = S.sn[last[u] + 1] - 1;
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const double t = evt_new[last[u]];
-            const uint8_t fo = evflags[last[u]];
-            if (fl[u] & EV_FIRST) {
-              tlo[u] = (fl[u] & EV_NOWRAP) ? 0.0 : t;
-              flo[u] = (fl[u] & EV_NOWRAP) ? (uint8_t)0 : fo;
-            }
-          }
+          root[u] = root_at(x);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -949,31 +943,29 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
           if ((x & ~63) >= end) break;  // (wave-uniform)
           bool f = false;
           if (x < m) {
-            const int spin = fl[u] >> 7, sig = 1 - 2 * spin;
-            const bool first = (fl[u] & EV_FIRST) != 0;
-            double len = 1.0;
-            int dw0 = 0, dw1 = 0;
-            if (!(fl[u] & EV_EMPTY)) {
-              len = (first && !(fl[u] & EV_NOWRAP)) ? ((thi[u] + 1.0) - tlo[u]) : (thi[u] - tlo[u]);
-              if (fl[u] & EV_SRC) { if (fl[u] & EV_DIR1) dw1 += sig; else dw0 += sig; }
-              if (flo[u] & EV_SRC) { if (flo[u] & EV_DIR1) dw1 -= sig; else dw0 -= sig; }
-            }
-            const int cls = (spin << 1) | ((fl[u] & EV_GAUGE) ? 1 : 0);
+            const int id = roots.rank(root[u]);
             if (!field) {
-              f = (cflip[id[u] >> 6] >> (id[u] & 63)) & 1;
-              seg_new[x] = (uint8_t)(spin ^ (int)f);
+              f = (((const uint32_t*)cflip)[id >> 5] >> (id & 31)) & 1;
+              seg_new[x] = (uint8_t)(((fl[u] >> 1) & 1) ^ (int)f);
             }
-            if (direct) {
-              ac.add(id[u], len, cls, first, dw0, dw1);
-            } else {
-              seg_len[x] = len;
-              seg_info[x] = (uint32_t)id[u] | ((uint32_t)cls << 24) | (first ? 1u << 26 : 0u) |
-                            ((uint32_t)(dw0 + 1) << 27) | ((uint32_t)(dw1 + 1) << 29);
-            }
+            if (!(fl[u] & SEG_FIRST)) account(x, id, thi[u] - tlo[u], fl[u], flo[u]);
           }
           const unsigned long long mk = __ballot(f);
           if (lane_id() == 0) nflip[x >> 6] = mk;
         }
+      }
+      // the sites' first segments: the segment below is the site's last (the
+      // line wraps through tau = 1), a virtual site's begins at tau = 0; the
+      // tau = 0 boundary counts with them
+      for (int s = tid; s < N; s += T) {
+        const int x = S.sn[s], last = S.sn[s + 1] - 1;
+        const int fx = evflags[x], fy = evflags[last];
+        const double tx = evt_new[x], ty = evt_new[last];
+        const int id = roots.rank(root_at(x));
+        const bool empty = (fx & SEG_EMPTY) != 0, nowrap = GEN && (fx & SEG_NOWRAP);
+        const double len = empty ? 1.0 : (nowrap ? tx : (tx + 1.0) - ty);
+        account(x, id, len, fx, empty ? fx : (nowrap ? 0 : fy));
+        if (direct) atomicAdd(&ac.n[id], 1ull << (16 * (fx & 3)));
       }
     }
     __syncthreads();
@@ -991,9 +983,11 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
         blk_each<4>(m, [&](int x) { return Seg{seg_info[x], seg_len[x]}; },
                     [&](int, const Seg& g) {
                       const int a = (int)(g.info & 0xffffffu) - w0;
-                      if ((unsigned)a < (unsigned)ac.W)
-                        ac.add(a, g.len, (int)(g.info >> 24) & 3, (g.info >> 26) & 1, (int)((g.info >> 27) & 3) - 1,
-                               (int)((g.info >> 29) & 3) - 1);
+                      if ((unsigned)a < (unsigned)ac.W) {
+                        const int cls = (int)(g.info >> 24) & 3;
+                        ac.add(a, g.len, cls, (int)((g.info >> 27) & 3) - 1, (int)((g.info >> 29) & 3) - 1);
+                        if ((g.info >> 26) & 1) atomicAdd(&ac.n[a], 1ull << (16 * cls));
+                      }
                     });
         __syncthreads();
       }
@@ -1004,7 +998,7 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
         if (i < wend) {
           ClusterAcc a;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) a.L[q] = ac.L[q * ac.W + i];
+          for (int q = 0; q < 4; ++q) a.L[q] = ac.L[4 * i + q];
           const unsigned long long cn = ac.n[i];
 #pragma unroll
           for (int q = 0; q < 4; ++q) a.n[q] = (int)((cn >> (16 * q)) & 0xffffu);
@@ -1047,7 +1041,7 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
         if (x < m) {
           const int id = direct ? roots.rank((int)p16[x]) : (int)(seg_info[x] & 0xffffffu);
           f = (cflip[id >> 6] >> (id & 63)) & 1;
-          seg_new[x] = (uint8_t)((evflags[x] >> 7) ^ (int)f);
+          seg_new[x] = (uint8_t)(((evflags[x] >> 1) & 1) ^ (int)f);
         }
         const unsigned long long mk = __ballot(f);
         if (lane_id() == 0) nflip[x >> 6] = mk;
