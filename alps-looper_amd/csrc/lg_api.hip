@@ -391,6 +391,7 @@ int Batch::init_exchange(const lg_params& p, const double* betas, int n, uint32_
   }
   if ((rc = reserve(cap, false))) return rc;
   params = ps;
+  swap_betas = true;
   if ((rc = set_layout(ds, std::vector<uint64_t>(n, 0)))) return rc;
   if ((rc = reset_state())) return rc;
   if ((rc = alloc(xslot, n)) || (rc = alloc(xbeta, n)) || (rc = alloc(xscale, n)) ||
@@ -511,8 +512,10 @@ int Batch::allocate(bool dynamic) {
   LG_HIP(hipMemset(scan_ctl, 0, 2 * sizeof(int)));
   // one workgroup per chain, except for server batches, whose mixes hold jobs
   // too large for it and whose sweeps replay the graph of each layout
+  if (!tile_prepare()) return set_error(LG_ERR_DEVICE, "the device refuses the tile kernel's LDS");
   blk_lds_grant = !dynamic && block_prepare() ? BLOCK_LDS_MAX : 0;
   if ((rc = alloc(col_part, (size_t)col_chunks(node_cap) * NUM_COLLECTOR_TERMS))) return rc;
+  if ((rc = alloc(pair_part, (size_t)col_chunks(node_cap) * PAIR_COLS))) return rc;
   if ((rc = alloc(totals, 2))) return rc;
   if ((rc = alloc(d_sweep, cap_chains))) return rc;
   if ((rc = alloc(rec_acc, (size_t)cap_chains * R_COUNT))) return rc;
@@ -604,6 +607,7 @@ int Batch::set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sw
   nbonds = (int)bonds;
   host_sweep = sweeps;
   choose_block();
+  choose_tiles();
   std::vector<int> bc(std::max(nbonds, 1)), sc(std::max(nsites, 1));
   std::vector<uint32_t> sw(std::max<size_t>(chains.size(), 1));
   for (size_t c = 0; c < chains.size(); ++c) {
@@ -686,6 +690,41 @@ int Batch::set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sw
   if (many_lists && c.link_cap == 1) c.link_cap = 0;
   if (has_extra_bonds()) c.link_cap = 0;  // in-site bonds, site operators: the per-operator kernel
   return apply_cfg(c);
+}
+
+// Tiles of the unions (k_tile_union, k_tile_cross), from 800000 segments on:
+// below that k_uf_union alone is faster, as its atomics do not queue yet and
+// it is one kernel (a sweep in us, tiles against none: chain L=128, beta=100
+// 89 and 79; square 48^2, beta=48 156 and 142; square 64^2, beta=64, of 612000
+// segments 197 and 199; chain L=1024, beta=1000, of 1.4M the unions alone 41
+// and 53).  A tile takes the segments' 256th part, 6144 to 15000: more of
+// them leave fewer unions to the kernel between tiles, up to two workgroups
+// for a CU's LDS (both kernels at square 128^2, beta=128: 10000 segments 125
+// us, 15000 107, 20000 100; square 256^2, beta=256: 611, 578, 659).
+void Batch::choose_tiles() {
+  // segments of a site: expected, and at most (an operator's weight is the
+  // bond's offset less its energy); the replicas of an exchange come to every
+  // temperature
+  std::vector<double> mean, most;
+  double segs = 0, mean_max = 0, most_max = 0;
+  for (size_t c = 0; c < chains.size(); ++c) {
+    const ChainDev& d = chains[c];
+    const lg_params& p = params[c];
+    mean.push_back(2 * expected_ops(p, d) / d.N);
+most.push_back(2 * d.beta / d.N * (d.offset_total + d.nb_real * (std::fabs(p.jz) / 4 + (d.L > 4 ? 0.32 : 0.5) * std::fabs(p.jxy))));
+    segs += mean[c] * d.N;
+    mean_max = std::max(mean_max, mean[c]);
+    most_max = std::max(most_max, most[c]);
+  }
+  ntiles = 0;
+  tile_cap = 0;
+  if (segs < 8e5) return;
+  const double target = std::min(15000.0, std::max(6144.0, segs / 256));
+  double per_bond = 0;
+  for (size_t c = 0; c < chains.size(); ++c) per_bond = std::max(per_bond, mean[c] * chains[c].N / 2 / chains[c].Nb);
+  cross_parts = (int)std::min(64.0, 1 + per_bond / 32);
+  for (size_t c = 0; c < chains.size(); ++c)
+    ntiles += set_tiles(chains[c], ntiles, swap_betas ? mean_max : mean[c], swap_betas ? most_max : most[c], target, tile_cap);
 }
 
 // Regions of the chains, and whether the batch takes one workgroup per chain.
@@ -934,13 +973,18 @@ DevBatch Batch::dev(int from) const {
   B.cand_t = cand_t; B.cand_g = cand_g; B.kc_new = kc_new;
   B.l0 = l0; B.l1 = l1; B.u0 = u0; B.u1 = u1; B.evflags = evflags; B.chain_node0 = chain_node0; B.node_site = node_site;
   B.parent = parent; B.fbit = fbit; B.fmask = fmask; B.rmask = rmask; B.acc = acc;
-  B.scan_status = scan_status; B.scan_ctl = scan_ctl; B.col_part = col_part; B.totals = totals; B.flags = flags;
+  B.scan_status = scan_status; B.scan_ctl = scan_ctl; B.col_part = col_part; B.pair_part = pair_part; B.totals = totals; B.flags = flags;
   B.sweep = d_sweep; B.rec_acc = rec_acc; B.rec_ring = rec_ring;
   B.ring_pos = ring_pos; B.end_count = end_count; B.ring_size = ring_size;
   B.any_field = 0;
   B.any_split = 0;
   B.any_extra = 0;
+  B.ntiles = ntiles;
+  B.cross_parts = cross_parts;
+  B.tile_cap = tile_cap;
+  B.pairs = 1;
   for (const auto& d : chains) {
+    if (d.L & 1) B.pairs = 0;
     if (d.h != 0.0) B.any_field = 1;
     if (d.nv > 1) B.any_split = 1;
     if (d.nb_real > d.nb_lat) B.any_extra |= 1;

@@ -101,6 +101,8 @@ struct ChainDev {
   // one workgroup per chain (lg_block.hip): the chain's own regions of the
   // operator and segment arrays
   int blk_op, blk_node, blk_opcap, blk_nodecap;
+  // unions by tiles (k_tile_union): the chain's first tile, sites and rows of one
+  int tile0, tile_w, tile_h;
 };
 // SSE chains: their sites' spins and bonds' counters are staged in LDS
 constexpr int SSE_MAX_SITES = 4096, SSE_MAX_BONDS = 4096;

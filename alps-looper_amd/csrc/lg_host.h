@@ -150,6 +150,7 @@ class Batch {
   int capture(int from);
   int check_flags();
   int flags_error() const;
+  void choose_tiles();
   void choose_block();
   int run_block(uint32_t n, uint32_t slot0);
   // st[cur] in the packed form (the chains' operators and segments consecutive)
@@ -184,6 +185,7 @@ class Batch {
   int scan_nparts = 0;
   int cus = 256;                  // compute units of the device
   double* col_part = nullptr;
+  double* pair_part = nullptr;
   int* totals = nullptr;
   int* flags = nullptr;
   uint32_t* d_sweep = nullptr;
@@ -211,6 +213,8 @@ class Batch {
   // faster form (blk_fit), unless launch settings were given (blk_off);
   // blk_regions: st[cur] stands in the chains' own regions
   bool blk_fit = false, blk_off = false, blk_regions = false, blk_general = false;
+  bool swap_betas = false;       // replica exchange: a chain comes to every temperature
+  int cross_parts = 1, ntiles = 0, tile_cap = 0;  // tiles of sites of the flat kernels' unions
   int blk_lds = 0, blk_threads = 0, blk_lds_grant = 0;
   double blk_us = 0;            // expected time of a sweep
   long long blk_exchange_ops = 0;  // operators of a region of an exchange batch

@@ -88,6 +88,10 @@ struct DevBatch {
   const int* sse_old;          // operator strings of the previous configuration (ChainDev::sse_base)
   int* sse_new;                // operator strings being built
   int* sse_perm;               // [ops] string position -> operator index of the new configuration
+  int pairs;                   // every bond joins sites of opposite gauge factors (every L is even): pairs of segments apart
+  double* pair_part;           // [col_chunks(node_cap)][PAIR_COLS] sums over the chunk's pairs
+  int cross_parts;             // parts of 32 operators of a bond
+  int ntiles, tile_cap;        // tiles of sites (ChainDev::tile0 ..) and segments that fit a tile's LDS
   const int* blk_nops;         // [nchains] operators per chain when each stands in its own region (else null)
 };
 
@@ -105,6 +109,12 @@ struct BlockArgs {
   double* seg_len;     // [nodes] a segment's length, and its cluster, class, tau = 0 and winding terms
   uint32_t* seg_info;
 };
+
+constexpr int PAIR_COLS = 3;
+constexpr int TILE_CAP_MAX = 36864;  // segments (144 KB of LDS, the tables aside)
+// dynamic LDS beyond 64 KB for the tile kernel; false where the device has none
+bool tile_prepare();
+int set_tiles(ChainDev& d, int first, double per_site, double most, double target, int& cap);
 
 struct LaunchCfg {
   int group = 64;              // lanes per bond in the diagonal update

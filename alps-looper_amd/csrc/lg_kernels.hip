@@ -689,46 +689,23 @@ __device__ __forceinline__ void rank_event(const DevBatch& B, const SiteLists& S
   }
 }
 
-// union-find on block-local segment indices in LDS (same hooking rule as
-// the global one: the larger root goes under the smaller)
-__device__ __forceinline__ int lds_find(int* P, int x) {
-  int p;
-  while ((p = __hip_atomic_load(P + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != x) x = p;
-  return x;
-}
-__device__ __forceinline__ void lds_unite(int* P, int a, int b) {
-  a = lds_find(P, a);
-  b = lds_find(P, b);
-  while (a != b) {
-    if (a < b) { int t = a; a = b; b = t; }
-    const int old = atomicCAS(P + a, a, b);
-    if (old == a) return;
-    a = lds_find(P, old);
-    b = lds_find(P, b);
-  }
-}
-
 // One block step handles SITES = 64 * WAVES / TPS consecutive sites, TPS
 // threads per site (several waves per site for long world lines, where one
 // wave would rank each list element by element; a quarter wave for short
-// ones, where a wave would idle most lanes).  Operators of a bond whose two sites
-// are both in the step ("inner" operators: neighbours along the fast lattice
-// direction) are united here in LDS, and each segment's parent is written as
-// its local root; k_uf_union skips them (u1 is stored complemented).  Roots
-// stay cluster minima, so the partition and every result are those of the
-// plain union-find.
+// ones, where a wave would idle most lanes).  Bound by the LDS searches' latency;
+// the unions are left to the kernels after it (with unions among the step's
+// sites, a third of the operators, it took 103 us at square 128^2, beta=128,
+// 85 without).
 constexpr int LINK_U = 4;  // staged elements per thread in flight
 
 template <int CAP, int WAVES, int TPS>
 __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
   if (overflowed(B)) return;
   constexpr int SITES = 64 * WAVES / TPS;
-  __shared__ double lt_all[SITES][CAP];           // staged times, list order; then local parents
-  __shared__ uint16_t lpre_all[SITES][CAP + 4];   // off-diagonal prefix counts; then element ranks
+  __shared__ double lt_all[SITES][CAP];           // staged times, list order
+  __shared__ uint16_t lpre_all[SITES][CAP + 4];   // off-diagonal prefix counts
   __shared__ uint16_t inv_all[SITES][CAP];        // rank -> staged element
   __shared__ uint8_t lfl_all[SITES][CAP];         // staged element -> event flags | spin below << 7
-  __shared__ int wn0[SITES], wn1[SITES], wtot[SITES], wnbd[SITES];
-  __shared__ int wbond[SITES][4], woff[SITES][4];
   // site slot of the step; with whole waves per site it is wave-uniform (read
   // as such, which keeps the site's list descriptors in scalar registers)
   const int w = TPS >= 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TPS) : (int)(threadIdx.x / TPS);
@@ -737,7 +714,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
   uint16_t* lpre = lpre_all[w];
   uint16_t* inv = inv_all[w];
   uint8_t* lfl = lfl_all[w];
-  int* lpar = reinterpret_cast<int*>(&lt_all[0][0]);  // SITES * CAP * 2 ints
+  const bool own_root = B.ntiles == 0;  // (k_tile_union writes the parents otherwise)
   int slo, shi;
   xcd_share(B.nsites, slo, shi);
   for (int g = slo; g < shi; g += SITES) {  // block-uniform steps
@@ -748,7 +725,6 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) { S.bond[j] = -1; S.off[j] = S.lo[j] = S.len[j] = S.side[j] = 0; }
     int tot = 0, s = 0, n0 = 0, n1 = 0;
-    int other[4] = {-1, -1, -1, -1};   // the bond's other site (global index)
     uint8_t spin0 = 0, gflag = 0;
     const ChainDev* Pp = nullptr;
     if (have) {
@@ -768,7 +744,6 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
         S.len[j] = B.bo_new[gb + 1] - S.lo[j];
         S.off[j] = tot;
         S.side[j] = (s0 == s) ? 0 : 1;
-        other[j] = P.site_base + ((s0 == s) ? s1 : s0);
         tot += S.len[j];
       }
       n0 = B.soff_new[gs];
@@ -820,32 +795,17 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
           lpre[off + j + len] = (uint16_t)(len > 0 ? v : 0);
         }
       }
-      if (sl == 0) {
-        wn0[w] = n0;
-        wn1[w] = n1;
-        wtot[w] = tot;
-        wnbd[w] = S.nbd;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { wbond[w][j] = S.bond[j]; woff[w][j] = S.off[j]; }
-      }
-    } else if (sl == 0) {
-      wtot[w] = -1;
     }
     __syncthreads();
-    // local unions need every site of the step staged and in one chain
-    bool inner_ok = true;
-    const int c0 = B.site_chain[g];
-    for (int v = 0; v < SITES; ++v)
-      if (g + v < shi && (wtot[v] > CAP || B.site_chain[g + v] != c0)) inner_ok = false;
     if (have && tot > 0) {
       const bool lds = tot <= CAP;
       for (int e = sl; e < tot; e += TPS) {
         // the element's list, selected with constant indices
-        int i = 0, offi = S.off[0], loi = S.lo[0], bi = S.bond[0], side = S.side[0], oth = other[0];
+        int i = 0, offi = S.off[0], loi = S.lo[0], bi = S.bond[0], side = S.side[0];
 #pragma unroll
         for (int j = 1; j < 4; ++j)
           if (j < S.nbd && e >= S.off[j]) {
-            i = j; offi = S.off[j]; loi = S.lo[j]; bi = S.bond[j]; side = S.side[j]; oth = other[j];
+            i = j; offi = S.off[j]; loi = S.lo[j]; bi = S.bond[j]; side = S.side[j];
           }
         const int p = e - offi;
         const int k = loi + p;
@@ -858,8 +818,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
         const uint8_t sp = spin0 ^ (uint8_t)(par & 1);
         const int node = n0 + rank;
         const int up = (node + 1 == n1) ? n0 : node + 1;  // segment above the event
-        const bool inner = inner_ok && oth >= g && oth < g + SITES && oth < shi;
-        if (side) { B.l1[k] = node; B.u1[k] = inner ? ~up : up; } else { B.l0[k] = node; B.u0[k] = up; }
+        if (side) { B.l1[k] = node; B.u1[k] = up; } else { B.l0[k] = node; B.u0[k] = up; }
         if (lds) {
           inv[rank] = (uint16_t)e;
           lfl[e] = (uint8_t)(fl | (sp << 7));  // flags use bits 0-5
@@ -867,13 +826,13 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
           B.evt_new[node] = tau;
           B.segspin_new[node] = sp;
           B.evflags[node] = fl;
-          B.parent[node] = node;
+          if (own_root) B.parent[node] = node;
           if (rank == 0) B.node_site[node] = gs;
         }
       }
     }
     __syncthreads();
-    // segment arrays in node order; element ranks for the local unions
+    // segment arrays in node order
     if (have && tot > 0 && tot <= CAP) {
       for (int r = sl; r < tot; r += TPS) {
         const int e = inv[r];
@@ -881,51 +840,9 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
         const uint8_t f = lfl[e];
         B.segspin_new[n0 + r] = f >> 7;
         B.evflags[n0 + r] = f & 0x7f;
+        if (own_root) B.parent[n0 + r] = n0 + r;
         if (r == 0) B.node_site[n0 + r] = gs;
-        lpre[e] = (uint16_t)r;
       }
-    }
-    __syncthreads();
-    // step's segments [N0, N1): local unions of the inner operators
-    const int last = min(g + SITES, shi) - 1 - g;
-    const int N0 = wn0[0], N1 = wn1[last];
-    if (inner_ok) {
-      for (int x = threadIdx.x; x < N1 - N0; x += blockDim.x) lpar[x] = x;
-      __syncthreads();
-      if (have && tot > 0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j >= S.nbd || S.side[j] != 0) continue;
-          const int wt = other[j] - g;
-          if (other[j] < g || wt >= SITES || other[j] >= shi) continue;
-          int jt = 0;
-          while (jt < 3 && wbond[wt][jt] != S.bond[j]) ++jt;
-          const uint16_t* rk_t = lpre_all[wt];
-          const int t0 = wn0[wt] - N0, t1 = wn1[wt] - N0, m0 = n0 - N0, m1 = n1 - N0;
-          for (int p = sl; p < S.len[j]; p += TPS) {
-            const int a0 = m0 + lpre[S.off[j] + p];
-            const int b0 = (a0 + 1 == m1) ? m0 : a0 + 1;
-            const int a1 = t0 + rk_t[woff[wt][jt] + p];
-            const int b1 = (a1 + 1 == t1) ? t0 : a1 + 1;
-            const int gr = (B.oi_new[S.lo[j] + p] >> 1) & 3;
-            if (gr & 2) {            // frozen: all four legs
-              lds_unite(lpar, a0, a1);
-              lds_unite(lpar, b0, b1);
-              lds_unite(lpar, a0, b0);
-            } else if (gr == 0) {    // horizontal cut
-              lds_unite(lpar, a0, a1);
-              lds_unite(lpar, b0, b1);
-            } else {                 // cross
-              lds_unite(lpar, a0, b1);
-              lds_unite(lpar, a1, b0);
-            }
-          }
-        }
-      }
-      __syncthreads();
-      for (int x = threadIdx.x; x < N1 - N0; x += blockDim.x) B.parent[N0 + x] = N0 + lds_find(lpar, x);
-    } else if (have && tot > 0 && tot <= CAP) {
-      for (int r = sl; r < tot; r += TPS) B.parent[n0 + r] = n0 + r;
     }
     __syncthreads();
   }
@@ -1170,27 +1087,235 @@ __global__ void __launch_bounds__(256) k_link_site(DevBatch B) {
   for (int gs = slo + threadIdx.x; gs < shi; gs += blockDim.x) link_site_events(B, gs);
 }
 
+// union-find on a tile's segments in LDS (same hooking rule as
+// the global one: the larger root goes under the smaller)
+__device__ __forceinline__ int lds_find(int* P, int x) {
+  int p;
+  while ((p = __hip_atomic_load(P + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != x) x = p;
+  return x;
+}
+__device__ __forceinline__ void lds_unite(int* P, int a, int b) {
+  a = lds_find(P, a);
+  b = lds_find(P, b);
+  while (a != b) {
+    if (a < b) { int t = a; a = b; b = t; }
+    const int old = atomicCAS(P + a, a, b);
+    if (old == a) return;
+    a = lds_find(P, old);
+    b = lds_find(P, b);
+  }
+}
+
+
+// Pairs.  Where two operators follow each other on a bond with no other event
+// between them on either site, and both have the horizontal graph, the two
+// segments between them are a cluster of their own: antiparallel, of one
+// length, without winding, without the tau = 0 boundary.  In a cold
+// antiferromagnet that is most clusters (square 48^2, beta=128: 87 % of them,
+// 26 % of the segments; chain L=512, beta=1000: 91 % and 52 %).  They need no
+// union, no accumulator and no collector: the lower of the two operators
+// marks both segments with their root and PAIR_NODE, and the estimator adds
+// their terms in registers (square 128^2, beta=128: k_estimate 177 -> 122 us, its
+// atomics 2.1M -> 0.76M; k_flip_collect 78 -> 56).  Sites of a bond have to have opposite gauge
+// factors (DevBatch::pairs: every L is even).
+constexpr int PAIR_NODE = (int)0x80000000;  // in DevBatch::parent
+constexpr int LDS_PAIR = 1 << 30;           // in a tile's local parents
+
+// An operator's legs, and whether the sides below and above it are a pair.
+struct OpLegs {
+  int info, l0, l1, u0, u1;
+  bool pair_below, pair_above;
+};
+__device__ __forceinline__ OpLegs op_legs(const DevBatch& B, int k, int nops) {
+  const int kp = max(k - 1, 0), kn = min(k + 1, nops - 1);
+  OpLegs o;
+  o.info = B.oi_new[k];
+  const int below = B.oi_new[kp], above = B.oi_new[kn];
+  o.l0 = B.l0[k]; o.l1 = B.l1[k]; o.u0 = B.u0[k]; o.u1 = B.u1[k];
+  const int nl0 = B.l0[kn], nl1 = B.l1[kn], pu0 = B.u0[kp], pu1 = B.u1[kp];
+  const bool can = B.pairs && ((o.info >> 1) & 3) == 0;
+  o.pair_below = can && kp != k && (below >> 1) == (o.info >> 1) && pu0 == o.l0 && pu1 == o.l1;
+  o.pair_above = can && kn != k && (above >> 1) == (o.info >> 1) && nl0 == o.u0 && nl1 == o.u1;
+  return o;
+}
+
+// An operator's unions by its graph, the legs as the caller numbers them.
+template <class Unite, class Mark>
+__device__ __forceinline__ void op_unions(const OpLegs& o, int l0, int l1, int u0, int u1, Unite unite, Mark mark) {
+  const int g = (o.info >> 1) & 3;
+  if (g & 2) {            // frozen: all four legs (graph_impl.h:282-283)
+    unite(l0, l1);
+    unite(u0, u1);
+    unite(l0, u0);
+  } else if (g == 0) {    // horizontal cut (graph_impl.h:284-288)
+    if (!o.pair_below) unite(l0, l1);
+    if (o.pair_above) mark(u0, u1);
+    else unite(u0, u1);
+  } else {                // cross (graph_impl.h:289-293)
+    unite(l0, u1);
+    unite(l1, u0);
+  }
+}
+
+// every operator, on the parents in memory
 __global__ void __launch_bounds__(256) k_uf_union(DevBatch B) {
   if (overflowed(B)) return;
   const int nops = B.totals[0];
   int klo, khi;
   xcd_share(nops, klo, khi);
   for (int k = klo + threadIdx.x; k < khi; k += blockDim.x) {
-    const int info = B.oi_new[k];
-    const int u1 = B.u1[k];
-    if (u1 < 0) continue;  // united in LDS by the linking kernel
-    const int l0 = B.l0[k], l1 = B.l1[k], u0 = B.u0[k];
-    const int g = (info >> 1) & 3;
-    if (g & 2) {            // frozen: all four legs (graph_impl.h:282-283)
-      uf_unite(B.parent, l0, l1);
-      uf_unite(B.parent, u0, u1);
-      uf_unite(B.parent, l0, u0);
-    } else if (g == 0) {    // horizontal cut (graph_impl.h:284-288)
-      uf_unite(B.parent, l0, l1);
-      uf_unite(B.parent, u0, u1);
-    } else {                // cross (graph_impl.h:289-293)
-      uf_unite(B.parent, l0, u1);
-      uf_unite(B.parent, l1, u0);
+    const OpLegs o = op_legs(B, k, nops);
+    op_unions(o, o.l0, o.l1, o.u0, o.u1, [&](int a, int b) { uf_unite(B.parent, a, b); },
+              [&](int a, int b) { B.parent[a] = B.parent[b] = min(a, b) | PAIR_NODE; });
+  }
+}
+
+// Unions by tiles of sites.  An atomic of a kernel that spans the chip goes to
+// memory (13 G/s: the unions of every operator are 1.9M of them, 137 us, at
+// square 128^2, beta=128), so a workgroup unites the operators within a tile
+// of sites in LDS first (37 us), and only the operators between tiles
+// (k_tile_cross: one in six; 0.6M atomics, 69 us) meet in memory, at the
+// tiles' roots.
+// A tile is tile_h rows of tile_w sites (ChainDev; near square, so that few
+// bonds leave it), its segments the rows' node ranges one after the other:
+// the local numbers ascend with the nodes, so the root of a part of a cluster
+// is its least node in both, and every result is that of the plain
+// union-find.  A tile whose segments do not fit the LDS it was planned for
+// (a configuration far from the expected one) unites in memory itself.
+constexpr int TILE_SITES = 256, TILE_ROWS = 16;  // at most (set_tiles)
+extern __shared__ int tile_par[];
+
+// the tile of a workgroup, consecutive tiles on one XCD
+struct Tile {
+  const ChainDev* P;
+  int W, H, per;       // the lattice's sites of a row and rows, bonds of a site
+  int x0, y0, h, w;    // first row and site, rows and sites of a row
+};
+__device__ __forceinline__ Tile this_tile(const DevBatch& B) {
+  const int x = blockIdx.x % NXCD, j = blockIdx.x / NXCD, q = B.ntiles / NXCD, r = B.ntiles % NXCD;
+  const int t = x * q + min(x, r) + j;
+  int c = 0;
+  for (int n = B.nchains; n > 1;) {
+    const int half = n >> 1;
+    if (B.chains[c + half].tile0 <= t) c += half;
+    n -= half;
+  }
+  Tile G;
+  G.P = B.chains + __builtin_amdgcn_readfirstlane(c);
+  const ChainDev& P = *G.P;
+  G.W = P.L;
+  G.H = P.kind == 0 ? 1 : P.L;
+  G.per = P.kind == 0 ? 1 : 2;
+  const int across = (G.W + P.tile_w - 1) / P.tile_w;
+  const int i = t - P.tile0, tx = i / across;
+  G.x0 = tx * P.tile_h;
+  G.y0 = (i - tx * across) * P.tile_w;
+  G.h = min(P.tile_h, G.H - G.x0);
+  G.w = min(P.tile_w, G.W - G.y0);
+  return G;
+}
+
+__global__ void __launch_bounds__(1024) k_tile_union(DevBatch B) {
+  if (overflowed(B)) return;
+  __shared__ int row_n[TILE_ROWS], row_at[TILE_ROWS + 1], row_k0[TILE_ROWS], row_k1[TILE_ROWS];
+  __shared__ int target[2 * TILE_SITES];
+  const int tid = threadIdx.x, T = blockDim.x;
+  const Tile G = this_tile(B);
+  const ChainDev& P = *G.P;
+  const int W = G.W, H = G.H, per = G.per, x0 = G.x0, y0 = G.y0, h = G.h, w = G.w;
+  if (tid < h) {
+    const int s = (x0 + tid) * W + y0, b = P.bond_base + per * s;
+    row_n[tid] = B.soff_new[P.site_base + s];
+    row_at[tid] = B.soff_new[P.site_base + s + w] - row_n[tid];
+    row_k0[tid] = B.bo_new[b];
+    row_k1[tid] = B.bo_new[b + per * w];
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int at = 0;
+    for (int r = 0; r < h; ++r) { const int m = row_at[r]; row_at[r] = at; at += m; }
+    row_at[h] = at;
+  }
+  __syncthreads();
+  const int M = row_at[h];
+  const bool lds = M <= B.tile_cap;
+  // the row that holds a bond's second site (-1: another tile's)
+  for (int i = tid; i < h * w * per; i += T) {
+    const int r = i / (w * per), j = i - r * (w * per);
+    int row;
+    if (per == 1 || (j & 1) == 0) row = (j / per + 1 < w || w == W) ? r : -1;
+    else row = r + 1 < h ? r + 1 : (h == H ? 0 : -1);
+    target[i] = row;
+  }
+  if (lds)
+    for (int x = tid; x < M; x += T) tile_par[x] = x;
+  // whole waves to the rows in turn
+  const int wave = tid >> 6, nwaves = T >> 6;
+  const int r0 = wave % h, share = (nwaves - r0 + h - 1) / h;  // (waves of this wave's first row)
+  auto rows = [&](auto body) {
+    if (nwaves >= h) body(r0, (wave / h) * 64 + lane_id(), share * 64);
+    else
+      for (int r = wave; r < h; r += nwaves) body(r, lane_id(), 64);
+  };
+  if (!lds) {
+    rows([&](int r, int i0, int step) {
+      for (int x = row_n[r] + i0; x < row_n[r] + row_at[r + 1] - row_at[r]; x += step) B.parent[x] = x;
+    });
+    __threadfence();
+  }
+  __syncthreads();
+  const int nops = B.totals[0];
+  rows([&](int r, int i0, int step) {
+    const int gb0 = P.bond_base + per * ((x0 + r) * W + y0), d0 = row_at[r] - row_n[r];
+    const int* const tg = target + r * w * per;
+    for (int k = row_k0[r] + i0; k < row_k1[r]; k += step) {
+      const OpLegs o = op_legs(B, k, nops);
+      const int row = tg[(o.info >> 3) - gb0];
+      if (row < 0) continue;
+      if (lds) {
+        const int d1 = row_at[row] - row_n[row];
+        op_unions(o, o.l0 + d0, o.l1 + d1, o.u0 + d0, o.u1 + d1, [&](int a, int b) { lds_unite(tile_par, a, b); },
+                  [&](int a, int b) { tile_par[a] = tile_par[b] = min(a, b) | LDS_PAIR; });
+      } else {
+        op_unions(o, o.l0, o.l1, o.u0, o.u1, [&](int a, int b) { uf_unite(B.parent, a, b); },
+                  [&](int a, int b) { B.parent[a] = B.parent[b] = min(a, b) | PAIR_NODE; });
+      }
+    }
+  });
+  if (!lds) return;
+  __syncthreads();
+  rows([&](int r, int i0, int step) {
+    for (int x = row_at[r] + i0; x < row_at[r + 1]; x += step) {
+      const int v = tile_par[x];
+      const int root = (v & LDS_PAIR) ? v & ~LDS_PAIR : lds_find(tile_par, v);
+      int row = r;
+      while (root < row_at[row]) --row;
+      B.parent[row_n[r] + (x - row_at[r])] = (row_n[row] + (root - row_at[row])) | ((v & LDS_PAIR) ? PAIR_NODE : 0);
+    }
+  });
+}
+
+// The operators between tiles: a workgroup takes the bonds that leave its tile
+// from the last site of every row and from the last row, 32 lanes a part of
+// a bond's operators (about one each: a lane's unions are a serial chain of
+// loads and atomics).  Bound by the atomics' rate: nearly every one is a hook
+// that some tile's root needs.
+constexpr int CROSS_LANES = 32;
+__global__ void __launch_bounds__(1024) k_tile_cross(DevBatch B) {
+  if (overflowed(B)) return;
+  const Tile G = this_tile(B);
+  const ChainDev& P = *G.P;
+  const int right = G.w == G.W ? 0 : G.h, down = G.H == 1 || G.h == G.H ? 0 : G.w;
+  const int parts = B.cross_parts, groups = blockDim.x / CROSS_LANES;
+  const int nops = B.totals[0];
+  for (int q = threadIdx.x / CROSS_LANES; q < (right + down) * parts; q += groups) {
+    const int e = q / parts, part = q - e * parts;
+    const int s = e < right ? (G.x0 + e) * G.W + G.y0 + G.w - 1 : (G.x0 + G.h - 1) * G.W + G.y0 + (e - right);
+    const int gb = P.bond_base + G.per * s + (e < right ? 0 : 1), end = B.bo_new[gb + 1];
+    for (int k = B.bo_new[gb] + part * CROSS_LANES + threadIdx.x % CROSS_LANES; k < end; k += parts * CROSS_LANES) {
+      const OpLegs o = op_legs(B, k, nops);
+      op_unions(o, o.l0, o.l1, o.u0, o.u1, [&](int a, int b) { uf_unite(B.parent, a, b); },
+                [&](int a, int b) { B.parent[a] = B.parent[b] = min(a, b) | PAIR_NODE; });
     }
   }
 }
@@ -1234,9 +1359,10 @@ __global__ void __launch_bounds__(256) k_uf_compress(DevBatch B) {
   xcd_share(M, ilo, ihi);
   for (int i = ilo + threadIdx.x; i < ihi; i += blockDim.x) {
     int p = B.parent[i];
+    if (p < 0) B.parent[i] = p &= ~PAIR_NODE;
     if (p != i) {
       int r = p, q;
-      while ((q = B.parent[r]) != r) r = q;
+      while ((q = B.parent[r] & ~PAIR_NODE) != r) r = q;
       B.parent[i] = r;
     } else {
       B.acc[i] = ClusterAcc{{0, 0, 0, 0}, {0, 0, 0, 0}, 0, 0};
@@ -1343,7 +1469,9 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
   __shared__ double hL[4][HT];
   __shared__ unsigned long long hw[HT];
   __shared__ unsigned int hn[2][HT];   // class counts: [0] = n0 | n1 << 16, [1] = n2 | n3 << 16
+  __shared__ double hpair[PAIR_COLS];
   const int tid = threadIdx.x;
+  if (tid < PAIR_COLS) hpair[tid] = 0;
   for (int s = tid; s < HT; s += EST_THREADS) {
     hkey[s] = -1;
     hL[0][s] = hL[1][s] = hL[2][s] = hL[3][s] = 0;
@@ -1360,6 +1488,10 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
   xcd_share(nchunks, clo, chi);
   for (int chunk = clo; chunk < chi; ++chunk) {
     const int cb = chain_of_node(B, min(chunk * echunk, M - 1));  // the chunk's first chain
+    // the chunk's pairs (of its first chain, whose record gets them in k_end_sweep)
+    const int cb_end = (cb + 1 < B.nchains) ? B.chain_node0[cb + 1] : M;
+    int npair = 0;
+    double pair_t2 = 0, pair_t = 0;
     // the thread's items in groups of EST_U: every memory step of a group
     // (parents, the walks to the roots, the segments' own data, the events
     // below them) is issued for all its items before any is waited for
@@ -1391,15 +1523,20 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
           flo[u] = B.evflags[pv];
         }
         uint32_t f[EST_U];
+        bool pair[EST_U];
         if (WALK) {
           // walks to the roots, one hop of every item at a time
           int p0[EST_U];
 #pragma unroll
-          for (int u = 0; u < EST_U; ++u) p0[u] = r[u];
+          for (int u = 0; u < EST_U; ++u) {
+            p0[u] = r[u];
+            pair[u] = r[u] < 0;
+            r[u] &= ~PAIR_NODE;
+          }
           for (bool more = true; more;) {
             int q[EST_U];
 #pragma unroll
-            for (int u = 0; u < EST_U; ++u) q[u] = B.parent[r[u]];
+            for (int u = 0; u < EST_U; ++u) q[u] = B.parent[r[u]] & ~PAIR_NODE;
             more = false;
 #pragma unroll
             for (int u = 0; u < EST_U; ++u)
@@ -1419,14 +1556,19 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
           }
         } else {
 #pragma unroll
-          for (int u = 0; u < EST_U; ++u) f[u] = B.fbit[r[u]];  // drawn for the root by k_uf_compress
+          for (int u = 0; u < EST_U; ++u) {
+            f[u] = B.fbit[r[u]];  // drawn for the root by k_uf_compress
+            pair[u] = false;
+          }
         }
         // flip and root bits of the wave's 64 consecutive nodes (the first a
         // multiple of 64), one word each, for the collector
 #pragma unroll
         for (int u = 0; u < EST_U; ++u) {
           const unsigned long long fm = __ballot(ok[u] && f[u] != 0);
-          const unsigned long long rm = __ballot(ok[u] && r[u] == nd[u]);
+          const bool root = ok[u] && r[u] == nd[u];
+          const unsigned long long rm = __ballot(root && !pair[u]);
+          npair += __popcll(__ballot(root && pair[u] && nd[u] < cb_end));
           const int w0 = __builtin_amdgcn_readfirstlane(ib) + u * EST_THREADS;
           if (lane_id() == 0 && g0 + u < items && w0 < M) {
             B.fmask[w0 >> 6] = fm;
@@ -1482,6 +1624,25 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
           if (first) B.spins_new[gs[u]] = (uint8_t)(spin ^ f[u]);
           B.segspin_new[i] = (uint8_t)(spin ^ f[u]);
           const int cls = (spin << 1) | ((fl[u] & EV_GAUGE) ? 1 : 0);  // seg_class
+          if (pair[u]) {
+            // both segments of a pair have this one's length and the classes
+            // cls and 3 - cls: ssize, umag and winding 0, usize the length,
+            // smag its value with a sign (cluster_terms)
+            if (r[u] == nd[u]) {
+              const double smag = (cls == 0 || cls == 3) ? len : -len;
+              if (i < cb_end) {
+                pair_t2 += len * len;
+                pair_t += smag;
+              } else {
+                double* rec = B.rec_acc + (size_t)chain_from(B, cb, i) * R_COUNT;
+                unsafeAtomicAdd(rec + term_slot(0), 1.0);
+                unsafeAtomicAdd(rec + term_slot(6), len * len);
+                unsafeAtomicAdd(rec + term_slot(14), len * len);
+                unsafeAtomicAdd(rec + term_slot(17), smag);
+              }
+            }
+            continue;
+          }
           double sL[4] = {0, 0, 0, 0};
           sL[cls] = len;
           ht_add(hkey, hL, hn, hw, B, r[u], sL, first ? (1 << (8 * cls)) : 0, pack_winding(dw0, dw1));
@@ -1490,8 +1651,18 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
       // the table goes to global memory every 256 * flush_items segments (at
       // the end of a group) and at the chunk's end; a block-uniform
       // condition, so every wave takes the barriers
-      if ((g0 + EST_U) % flush_every != 0 && g0 + EST_U < items) continue;
+      const bool last = g0 + EST_U >= items;
+      if ((g0 + EST_U) % flush_every != 0 && !last) continue;
+      if (last && B.pairs) {
+        const double v[PAIR_COLS] = {(double)npair, wave_sum_d(pair_t2), wave_sum_d(pair_t)};
+        if (lane_id() == 0 && npair > 0)
+          for (int q = 0; q < PAIR_COLS; ++q) atomicAdd(&hpair[q], v[q]);
+      }
       __syncthreads();
+      if (last && B.pairs && tid < PAIR_COLS) {
+        B.pair_part[(size_t)chunk * PAIR_COLS + tid] = hpair[tid];
+        hpair[tid] = 0;
+      }
       for (int s = tid; s < HT; s += EST_THREADS) {
         const int r = hkey[s];
         if (r < 0) continue;
@@ -1736,6 +1907,14 @@ __global__ void __launch_bounds__(END_THREADS) k_end_sweep(DevBatch B) {
     const int j0 = (start + cchunk - 1) / cchunk, j1 = (end + cchunk - 1) / cchunk;
     for (int j = j0 + tid; j < j1; j += END_THREADS)
       for (int q = 0; q < NCOL; ++q) v[q] += B.col_part[(size_t)j * NCOL + q];
+    if (B.pairs)  // the estimator's pairs, by the same chunks: clusters, usize^2 and smag^2, smag
+      for (int j = j0 + tid; j < j1; j += END_THREADS) {
+        const double* p = B.pair_part + (size_t)j * PAIR_COLS;
+        v[0] += p[0];
+        v[6] += p[1];
+        v[14] += p[1];
+        v[17] += p[2];
+      }
   }
 #pragma unroll
   for (int q = 0; q < NCOL; ++q) v[q] = wave_sum_d(v[q]);
@@ -1846,8 +2025,7 @@ __device__ __forceinline__ int element_node(const DevBatch& B, const ChainDev& P
   if (leg == 0) return B.l0[kg];
   if (leg == 1) return B.l1[kg];
   if (leg == 2) return B.u0[kg];
-  const int u1 = B.u1[kg];
-  return u1 < 0 ? ~u1 : u1;  // complemented: united in LDS
+  return B.u1[kg];
 }
 
 __global__ void k_canon_min(DevBatch B, int chain, int nelem, int* canon) {
@@ -1921,6 +2099,34 @@ static inline void mark(hipEvent_t* ev, int i, hipStream_t st) {
   if (ev) (void)hipEventRecord(ev[i], st);
 }
 
+bool tile_prepare() {
+  return hipFuncSetAttribute((const void*)k_tile_union, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             TILE_CAP_MAX * (int)sizeof(int)) == hipSuccess;
+}
+
+// Tiles for a chain whose sites hold per_site segments (at most `most`), about
+// `target` segments in one; its first tile is `first`.  Returns their number
+// and raises cap to the LDS a tile may take.
+int set_tiles(ChainDev& d, int first, double per_site, double most, double target, int& cap) {
+  const int W = d.L, H = d.kind == 0 ? 1 : d.L;
+  const int area = (int)std::min<double>(TILE_SITES, std::max(1.0, target / std::max(per_site, 1.0)));
+  int w = area, h = 1;
+  if (H > 1) {
+    while ((h + 1) * (h + 1) <= area && h < TILE_ROWS) ++h;
+    h = std::min(h, H);
+    w = area / h;
+  }
+  w = std::min(w, W);
+  // tiles of about one size
+  const int across = (W + w - 1) / w, down = (H + h - 1) / h;
+  d.tile_w = (W + across - 1) / across;
+  d.tile_h = (H + down - 1) / down;
+  d.tile0 = first;
+  const double full = d.tile_w * d.tile_h * std::max(most, 1.0);
+  cap = std::max(cap, (int)std::min<double>(TILE_CAP_MAX, full + 6 * std::sqrt(full) + 64));
+  return ((W + d.tile_w - 1) / d.tile_w) * ((H + d.tile_h - 1) / d.tile_h);
+}
+
 static void launch_sweep_sse(const DevBatch& B, const LaunchCfg& L, hipStream_t st, hipEvent_t* ev) {
   mark(ev, 0, st);
   launch_sse_walk(B, st);  // also the scan's epoch
@@ -1981,7 +2187,12 @@ void launch_cluster_stage(const DevBatch& B, const LaunchCfg& L, hipStream_t st,
     hipLaunchKernelGGL(k_boundary, dim3(blocks), dim3(256), 0, st, B);
   }
   // (the per-operator linking kernel unites as it links)
-  if (L.link_cap != 0) hipLaunchKernelGGL(k_uf_union, dim3(L.blocks_op), dim3(256), 0, st, B);
+  if (L.link_cap == 1 || (L.link_cap > 1 && B.ntiles == 0)) {
+    hipLaunchKernelGGL(k_uf_union, dim3(L.blocks_op), dim3(256), 0, st, B);
+  } else if (L.link_cap > 1) {
+    hipLaunchKernelGGL(k_tile_union, dim3(B.ntiles), dim3(B.tile_cap > 4096 ? 1024 : 256), B.tile_cap * sizeof(int), st, B);
+    hipLaunchKernelGGL(k_tile_cross, dim3(B.ntiles), dim3(B.tile_cap > 4096 ? 1024 : 256), 0, st, B);
+  }
   mark(ev, 2, st);
   if (L.compress) {
     hipLaunchKernelGGL(k_uf_compress, dim3(L.blocks_node), dim3(256), 0, st, B);

@@ -171,6 +171,10 @@ DevBatch na_dev(unsigned char* base, int N, int Nb, bool field) {
   B.any_field = field ? 1 : 0;
   B.any_split = 0;
   B.any_extra = 0;
+  B.pairs = 0;
+  B.pair_part = nullptr;
+  B.ntiles = B.tile_cap = 0;
+  B.cross_parts = 1;
   B.nslots = 0;
   B.op_cap = (int)NA_OPS;
   B.node_cap = (int)NA_NODES;
