@@ -852,54 +852,25 @@ __global__ void __launch_bounds__(64 * WAVES) k_link(DevBatch B) {
 // (c) lock-free union-find on segments: hook the larger root under the
 // smaller with atomicCAS, so every root is its cluster's minimum node (the
 // hooking rule of ECL-CC, Jaiganesh & Burtscher, HPDC'18).  parent[x] <= x
-// always holds.
+// always holds.  The linking kernels write every segment as its own parent.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int ld_parent(int* P, int x) {
   return __hip_atomic_load(P + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Plain walk to the root: shortening the path with stores while walking cost
-// more write traffic than the longer walks it saves (k_estimate points every
-// node at its root once all unions are done).
-__device__ __forceinline__ int uf_find(int* P, int v) {
-  int cur = v, next;
-  while (cur != (next = ld_parent(P, cur))) cur = next;
-  return cur;
-}
-
-__device__ __forceinline__ void uf_unite(int* P, int a, int b) {
-  int ra = uf_find(P, a), rb = uf_find(P, b);
-  while (ra != rb) {
-    if (ra < rb) { int t = ra; ra = rb; rb = t; }
-    // ra > rb: hook ra under rb
-    int old = atomicCAS(P + ra, ra, rb);
-    if (old == ra) return;
-    ra = uf_find(P, old);
-    rb = uf_find(P, rb);
-  }
-}
-
-// every segment its own root, before the unions of k_link_ops
-__global__ void __launch_bounds__(256) k_node_init(DevBatch B) {
-  if (overflowed(B)) return;
-  const int M = B.totals[1];
-  int ilo, ihi;
-  xcd_share(M, ilo, ihi);
-  for (int i = ilo + threadIdx.x; i < ihi; i += blockDim.x) B.parent[i] = i;
-}
-
 // Linking, one thread per operator: for each leg, the rank of the event on
 // its site by binary search in the site's other bond lists (global memory).
 // Used when sites hold few events (a wave per site would idle most lanes).
-// The thread then unites its operator's legs by its graph (the k_uf_union
-// rules) right away: k_node_init made every segment a root beforehand, and
-// the linking itself writes no parent, so the unions of different threads
-// only meet in the lock-free union-find.  This saves the separate union
-// pass, which re-read the four legs and the type of every operator.
 // EXTRA: some chain has bonds beyond the lattice's (in-site bonds of the
 // single-ion term: two legs, no bond vector; site operators of the
 // transverse field); a separate instance, so that the plain one carries
 // none of their tests.
+// With one virtual site a real site, a site has at most five lists, and the
+// lists of both sites are searched together, a step of each at a time: a
+// thread's work is a chain of dependent loads, which the searches one after
+// the other made eight or ten times as long (square 32^2 in a transverse
+// field, 14000 operators: 46 us with the unions in it; 9 us, and 28 for the
+// unions by k_uf_union).
 template <bool EXTRA>
 __global__ void __launch_bounds__(256) k_link_ops(DevBatch B) {
   if (overflowed(B)) return;
@@ -912,16 +883,96 @@ __global__ void __launch_bounds__(256) k_link_ops(DevBatch B) {
     const ChainDev& P = B.chains[B.bond_chain[gb]];
     const int b = gb - P.bond_base;
     const double tau = B.ot_new[k];
-    const int r = k - B.bo_new[gb];
+    const int r = k - B.bo_new[gb], kpar = B.kc_new[k];
     // a site operator (transverse field): one event, on its site, with no
     // bond vector (no source flag), and no union: the world line is cut
     const bool site = EXTRA && b >= P.nb_real;
     const bool lattice = !EXTRA || b < P.nb_lat;  // bonds with a bond vector
     const uint8_t dflag = (lattice && bond_dir(P, b)) ? EV_DIR1 : 0;
-    int s0, s1;
-    if (EXTRA) op_sites(P, b, s0, s1);
-    else bond_sites(P, b, s0, s1);
+    int sites[2];
+    if (EXTRA) op_sites(P, b, sites[0], sites[1]);
+    else bond_sites(P, b, sites[0], sites[1]);
     int lo_leg[2], up_leg[2];  // lower and upper segment of each side
+    int rank[2], par[2];       // the event's rank on its site, the off-diagonal operators below it there
+    if (P.nv == 1) {
+      constexpr int NL = EXTRA ? 5 : 4;
+      int at[2 * NL], len[2 * NL], first[2 * NL], all[2 * NL];
+      bool ties[2 * NL];
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        int bl[NL];
+        const int nbd = site_bonds(P, sites[side], bl);
+        if (EXTRA) bl[NL - 1] = P.Nb > P.nb_real ? P.nb_real + sites[side] : b;  // the site's own operators
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+          const int q = side * NL + i;
+          // (its own list, and those it does not have: empty)
+          const int bp = (EXTRA && i == NL - 1) || i < nbd ? bl[i] : b;
+          const int lo = B.bo_new[P.bond_base + bp], hi = B.bo_new[P.bond_base + bp + 1];
+          first[q] = at[q] = lo;
+          all[q] = len[q] = bp == b || (EXTRA && side && site) ? 0 : hi - lo;
+          ties[q] = bp < b;
+        }
+      }
+      for (bool more = true; more;) {
+        double t[2 * NL];
+#pragma unroll
+        for (int q = 0; q < 2 * NL; ++q) t[q] = B.ot_new[len[q] > 0 ? at[q] + (len[q] >> 1) : k];
+        more = false;
+#pragma unroll
+        for (int q = 0; q < 2 * NL; ++q) {
+          const int h = len[q] >> 1;
+          const bool below = len[q] > 0 && (ties[q] ? t[q] <= tau : t[q] < tau);
+          at[q] += below ? h + 1 : 0;
+          len[q] = below ? len[q] - h - 1 : h;
+          more |= len[q] > 0;
+        }
+      }
+      int kc[2 * NL], oi[2 * NL];
+#pragma unroll
+      for (int q = 0; q < 2 * NL; ++q) {
+        const int x = all[q] > 0 ? min(at[q], first[q] + all[q] - 1) : k;
+        kc[q] = B.kc_new[x];
+        oi[q] = B.oi_new[x];
+      }
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        rank[side] = r;
+        par[side] = kpar;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+          const int q = side * NL + i, n = at[q] - first[q];
+          if (all[q] == 0) continue;
+          rank[side] += n;
+          par[side] += kc[q] + (n == all[q] ? oi[q] & 1 : 0);
+        }
+      }
+    } else {  // virtual sites: list by list
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        rank[side] = r;
+        par[side] = kpar;
+        if (side && site) continue;
+        const int s = sites[side];
+        // the event's rank among the site's other lists (ties by bond index)
+        // and the off-diagonal operators below it there
+        auto other_list = [&](int bp) {
+          if (bp == b) return;
+          const int gbp = P.bond_base + bp;
+          const int lo = B.bo_new[gbp], hi = B.bo_new[gbp + 1];
+          const int q = (bp < b) ? upper_bound_d(B.ot_new + lo, hi - lo, tau) : lower_bound_d(B.ot_new + lo, hi - lo, tau);
+          rank[side] += q;
+          if (q < hi - lo) par[side] += B.kc_new[lo + q];
+          else if (hi > lo) par[side] += B.kc_new[hi - 1] + (B.oi_new[hi - 1] & 1);
+        };
+        const int nbd = site_lists(P);
+        for (int i = 0; i < nbd; ++i) other_list(site_bond(P, s, i));
+        if (EXTRA) {
+          for (int j = 0, nd = P.npair > 0 ? P.nv - 1 : 0; j < nd; ++j) other_list(dpair_bond(P, s, j));  // nv - 1 in-site lists
+          if (P.Nb > P.nb_real) other_list(P.nb_real + s);                            // the site's own operators
+        }
+      }
+    }
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       if (side && site) {
@@ -929,70 +980,28 @@ __global__ void __launch_bounds__(256) k_link_ops(DevBatch B) {
         B.u1[k] = up_leg[0];
         break;
       }
-      const int s = side ? s1 : s0;
-      int rank = r;
-      int par = B.kc_new[k];
-      // the event's rank among the site's other lists (ties by bond index)
-      // and the off-diagonal operators below it there
-      auto other_list = [&](int bp) {
-        if (bp == b) return;
-        const int gbp = P.bond_base + bp;
-        const int lo = B.bo_new[gbp], hi = B.bo_new[gbp + 1];
-        const int q = (bp < b) ? upper_bound_d(B.ot_new + lo, hi - lo, tau) : lower_bound_d(B.ot_new + lo, hi - lo, tau);
-        rank += q;
-        if (q < hi - lo) par += B.kc_new[lo + q];
-        else if (hi > lo) par += B.kc_new[hi - 1] + (B.oi_new[hi - 1] & 1);
-      };
-      if (P.nv == 1) {
-        int bl[4];
-        const int nbd = site_bonds(P, s, bl);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (i >= nbd) break;
-          other_list(bl[i]);
-        }
-      } else {  // virtual sites: up to eight lists
-        const int nbd = site_lists(P);
-        for (int i = 0; i < nbd; ++i) other_list(site_bond(P, s, i));
-      }
-      if (EXTRA) {
-        for (int j = 0, nd = P.npair > 0 ? P.nv - 1 : 0; j < nd; ++j) other_list(dpair_bond(P, s, j));  // nv - 1 in-site lists
-        if (P.Nb > P.nb_real) other_list(P.nb_real + s);                            // the site's own operators
-      }
-      const int gs = P.site_base + s;
+      const int gs = P.site_base + sites[side];
       const int n0 = B.soff_new[gs], n1 = B.soff_new[gs + 1];
-      const int node = n0 + rank;
+      const int node = n0 + rank[side];
       const bool split = P.nv > 1;
       const int up = (node + 1 == n1) ? n0 : node + 1;  // segment above the event (split: never wraps)
-      const uint8_t gflag = gauge(P, s) < 0 ? EV_GAUGE : 0;
-      const uint8_t sp = B.spins_old[P.old_site_base + s] ^ (uint8_t)(par & 1);
+      const uint8_t gflag = gauge(P, sites[side]) < 0 ? EV_GAUGE : 0;
+      const uint8_t sp = B.spins_old[P.old_site_base + sites[side]] ^ (uint8_t)(par[side] & 1);
       B.evt_new[node] = tau;
       B.segspin_new[node] = sp;
-      B.evflags[node] = (uint8_t)((info & 1) | ((side || !lattice) ? 0 : EV_SRC) | dflag | (rank == 0 ? EV_FIRST : 0) |
-                                  gflag | (split && rank == 0 ? EV_NOWRAP : 0));
-      if (rank == 0) B.node_site[node] = gs;
+      B.evflags[node] = (uint8_t)((info & 1) | ((side || !lattice) ? 0 : EV_SRC) | dflag | (rank[side] == 0 ? EV_FIRST : 0) |
+                                  gflag | (split && rank[side] == 0 ? EV_NOWRAP : 0));
+      B.parent[node] = node;
+      if (rank[side] == 0) B.node_site[node] = gs;
       if (split && up == n1 - 1) {  // the last event: the site's top segment, up to tau = 1
         B.evt_new[up] = 1.0;
         B.segspin_new[up] = sp ^ (uint8_t)(info & 1);
         B.evflags[up] = gflag;
+        B.parent[up] = up;
       }
       if (side) { B.l1[k] = node; B.u1[k] = up; } else { B.l0[k] = node; B.u0[k] = up; }
       lo_leg[side] = node;
       up_leg[side] = up;
-    }
-    if (site) continue;
-    const int g = (info >> 1) & 3;
-    const int l0 = lo_leg[0], u0 = up_leg[0], l1 = lo_leg[1], u1 = up_leg[1];
-    if (g & 2) {            // frozen: all four legs (graph_impl.h:282-283)
-      uf_unite(B.parent, l0, l1);
-      uf_unite(B.parent, u0, u1);
-      uf_unite(B.parent, l0, u0);
-    } else if (g == 0) {    // horizontal cut (graph_impl.h:284-288)
-      uf_unite(B.parent, l0, l1);
-      uf_unite(B.parent, u0, u1);
-    } else {                // cross (graph_impl.h:289-293)
-      uf_unite(B.parent, l0, u1);
-      uf_unite(B.parent, l1, u0);
     }
   }
 }
@@ -1087,26 +1096,6 @@ __global__ void __launch_bounds__(256) k_link_site(DevBatch B) {
   for (int gs = slo + threadIdx.x; gs < shi; gs += blockDim.x) link_site_events(B, gs);
 }
 
-// union-find on a tile's segments in LDS (same hooking rule as
-// the global one: the larger root goes under the smaller)
-__device__ __forceinline__ int lds_find(int* P, int x) {
-  int p;
-  while ((p = __hip_atomic_load(P + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != x) x = p;
-  return x;
-}
-__device__ __forceinline__ void lds_unite(int* P, int a, int b) {
-  a = lds_find(P, a);
-  b = lds_find(P, b);
-  while (a != b) {
-    if (a < b) { int t = a; a = b; b = t; }
-    const int old = atomicCAS(P + a, a, b);
-    if (old == a) return;
-    a = lds_find(P, old);
-    b = lds_find(P, b);
-  }
-}
-
-
 // Pairs.  Where two operators follow each other on a bond with no other event
 // between them on either site, and both have the horizontal graph, the two
 // segments between them are a cluster of their own: antiparallel, of one
@@ -1120,6 +1109,56 @@ __device__ __forceinline__ void lds_unite(int* P, int a, int b) {
 // factors (DevBatch::pairs: every L is even).
 constexpr int PAIR_NODE = (int)0x80000000;  // in DevBatch::parent
 constexpr int LDS_PAIR = 1 << 30;           // in a tile's local parents
+
+// A union-find's parents: in memory, or a tile's segments in LDS.  SHORTEN:
+// walks leave each node they pass at its grandparent (a node with a parent
+// always has an ancestor for one, and only roots are hooked, so the store
+// loses nothing).
+template <bool SHORTEN>
+struct MemParents {
+  int* p;
+  __device__ __forceinline__ int find(int x) const {
+    int q = ld_parent(p, x);
+    while (q != x) {
+      const int r = ld_parent(p, q);
+      if (r == q) return q;
+      if (SHORTEN) {
+        __hip_atomic_store(p + x, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        x = r;
+        q = ld_parent(p, x);
+      } else {
+        x = q;
+        q = r;
+      }
+    }
+    return x;
+  }
+  __device__ __forceinline__ int hook(int a, int b) const { return atomicCAS(p + a, a, b); }
+  __device__ __forceinline__ void pair(int a, int b) const { p[a] = p[b] = min(a, b) | PAIR_NODE; }
+};
+struct LdsParents {
+  int* p;
+  __device__ __forceinline__ int find(int x) const {
+    int q;
+    while ((q = __hip_atomic_load(p + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != x) x = q;
+    return x;
+  }
+  __device__ __forceinline__ int hook(int a, int b) const { return atomicCAS(p + a, a, b); }
+  __device__ __forceinline__ void pair(int a, int b) const { p[a] = p[b] = min(a, b) | LDS_PAIR; }
+};
+
+template <class U>
+__device__ __forceinline__ void unite(const U& u, int a, int b) {
+  a = u.find(a);
+  b = u.find(b);
+  while (a != b) {
+    if (a < b) { const int t = a; a = b; b = t; }
+    const int old = u.hook(a, b);  // the larger root under the smaller
+    if (old == a) return;
+    a = u.find(old);
+    b = u.find(b);
+  }
+}
 
 // An operator's legs, and whether the sides below and above it are a pair.
 struct OpLegs {
@@ -1139,34 +1178,46 @@ __device__ __forceinline__ OpLegs op_legs(const DevBatch& B, int k, int nops) {
   return o;
 }
 
-// An operator's unions by its graph, the legs as the caller numbers them.
-template <class Unite, class Mark>
-__device__ __forceinline__ void op_unions(const OpLegs& o, int l0, int l1, int u0, int u1, Unite unite, Mark mark) {
+// An operator's unions by its graph (graph_impl.h:277-295), the legs as the
+// caller numbers them.
+template <class U>
+__device__ __forceinline__ void op_unions(const U& u, const OpLegs& o, int l0, int l1, int u0, int u1) {
   const int g = (o.info >> 1) & 3;
-  if (g & 2) {            // frozen: all four legs (graph_impl.h:282-283)
-    unite(l0, l1);
-    unite(u0, u1);
-    unite(l0, u0);
-  } else if (g == 0) {    // horizontal cut (graph_impl.h:284-288)
-    if (!o.pair_below) unite(l0, l1);
-    if (o.pair_above) mark(u0, u1);
-    else unite(u0, u1);
-  } else {                // cross (graph_impl.h:289-293)
-    unite(l0, u1);
-    unite(l1, u0);
+  if (g & 2) {            // frozen: all four legs
+    unite(u, l0, l1);
+    unite(u, u0, u1);
+    unite(u, l0, u0);
+  } else if (g == 0) {    // horizontal cut
+    if (!o.pair_below) unite(u, l0, l1);
+    if (o.pair_above) u.pair(u0, u1);
+    else unite(u, u0, u1);
+  } else {                // cross
+    unite(u, l0, u1);
+    unite(u, l1, u0);
   }
 }
 
-// every operator, on the parents in memory
+// Every operator, on the parents in memory.  EXTRA: some chain has in-site
+// bonds, whose two sites have one gauge factor, or site operators.  Those
+// models freeze the segments of whole neighbourhoods together, whose trees are
+// deep: walks that shorten them pay there (square 32^2 in a transverse field:
+// 31 -> 28 us, and k_estimate, which walks after it, 19 -> 13), but not
+// elsewhere (square 256^2, beta=8: 291 -> 305 us a sweep).
+template <bool EXTRA>
 __global__ void __launch_bounds__(256) k_uf_union(DevBatch B) {
   if (overflowed(B)) return;
   const int nops = B.totals[0];
   int klo, khi;
   xcd_share(nops, klo, khi);
   for (int k = klo + threadIdx.x; k < khi; k += blockDim.x) {
-    const OpLegs o = op_legs(B, k, nops);
-    op_unions(o, o.l0, o.l1, o.u0, o.u1, [&](int a, int b) { uf_unite(B.parent, a, b); },
-              [&](int a, int b) { B.parent[a] = B.parent[b] = min(a, b) | PAIR_NODE; });
+    OpLegs o = op_legs(B, k, nops);
+    if (EXTRA) {
+      const ChainDev& P = B.chains[B.bond_chain[o.info >> 3]];
+      const int b = (o.info >> 3) - P.bond_base;
+      if (b >= P.nb_real) continue;  // a site operator cuts the world line
+      if (b >= P.nb_lat) o.pair_below = o.pair_above = false;
+    }
+    op_unions(MemParents<EXTRA>{B.parent}, o, o.l0, o.l1, o.u0, o.u1);
   }
 }
 
@@ -1274,11 +1325,9 @@ __global__ void __launch_bounds__(1024) k_tile_union(DevBatch B) {
       if (row < 0) continue;
       if (lds) {
         const int d1 = row_at[row] - row_n[row];
-        op_unions(o, o.l0 + d0, o.l1 + d1, o.u0 + d0, o.u1 + d1, [&](int a, int b) { lds_unite(tile_par, a, b); },
-                  [&](int a, int b) { tile_par[a] = tile_par[b] = min(a, b) | LDS_PAIR; });
+        op_unions(LdsParents{tile_par}, o, o.l0 + d0, o.l1 + d1, o.u0 + d0, o.u1 + d1);
       } else {
-        op_unions(o, o.l0, o.l1, o.u0, o.u1, [&](int a, int b) { uf_unite(B.parent, a, b); },
-                  [&](int a, int b) { B.parent[a] = B.parent[b] = min(a, b) | PAIR_NODE; });
+        op_unions(MemParents<false>{B.parent}, o, o.l0, o.l1, o.u0, o.u1);
       }
     }
   });
@@ -1287,7 +1336,7 @@ __global__ void __launch_bounds__(1024) k_tile_union(DevBatch B) {
   rows([&](int r, int i0, int step) {
     for (int x = row_at[r] + i0; x < row_at[r + 1]; x += step) {
       const int v = tile_par[x];
-      const int root = (v & LDS_PAIR) ? v & ~LDS_PAIR : lds_find(tile_par, v);
+      const int root = (v & LDS_PAIR) ? v & ~LDS_PAIR : LdsParents{tile_par}.find(v);
       int row = r;
       while (root < row_at[row]) --row;
       B.parent[row_n[r] + (x - row_at[r])] = (row_n[row] + (root - row_at[row])) | ((v & LDS_PAIR) ? PAIR_NODE : 0);
@@ -1314,8 +1363,7 @@ __global__ void __launch_bounds__(1024) k_tile_cross(DevBatch B) {
     const int gb = P.bond_base + G.per * s + (e < right ? 0 : 1), end = B.bo_new[gb + 1];
     for (int k = B.bo_new[gb] + part * CROSS_LANES + threadIdx.x % CROSS_LANES; k < end; k += parts * CROSS_LANES) {
       const OpLegs o = op_legs(B, k, nops);
-      op_unions(o, o.l0, o.l1, o.u0, o.u1, [&](int a, int b) { uf_unite(B.parent, a, b); },
-                [&](int a, int b) { B.parent[a] = B.parent[b] = min(a, b) | PAIR_NODE; });
+      op_unions(MemParents<false>{B.parent}, o, o.l0, o.l1, o.u0, o.u1);
     }
   }
 }
@@ -1345,7 +1393,7 @@ __global__ void __launch_bounds__(256) k_boundary(DevBatch B) {
         es |= (uint32_t)B.segspin_new[top[a]] << a;
       }
     }
-    join_boundary(P, B.sweep[c], r, bot, top, bs, es, [&](int a, int b) { uf_unite(B.parent, a, b); });
+    join_boundary(P, B.sweep[c], r, bot, top, bs, es, [&](int a, int b) { unite(MemParents<false>{B.parent}, a, b); });
   }
 }
 
@@ -2165,7 +2213,6 @@ void launch_cluster_stage(const DevBatch& B, const LaunchCfg& L, hipStream_t st,
   // 1536-event kernel keeps the per-node grid (square 512^2, beta=512: 5.76
   // ms at 8 steps per block, 5.95 at one)
   if (L.link_cap == 0) {
-    hipLaunchKernelGGL(k_node_init, dim3(L.blocks_node), dim3(256), 0, st, B);
     if (B.any_extra) hipLaunchKernelGGL(k_link_ops<true>, dim3(L.blocks_op), dim3(256), 0, st, B);
     else hipLaunchKernelGGL(k_link_ops<false>, dim3(L.blocks_op), dim3(256), 0, st, B);
   } else if (L.link_cap == 1) {
@@ -2186,10 +2233,10 @@ void launch_cluster_stage(const DevBatch& B, const LaunchCfg& L, hipStream_t st,
     const int blocks = max(1, min(L.blocks_op, (B.nsites + 255) / 256));
     hipLaunchKernelGGL(k_boundary, dim3(blocks), dim3(256), 0, st, B);
   }
-  // (the per-operator linking kernel unites as it links)
-  if (L.link_cap == 1 || (L.link_cap > 1 && B.ntiles == 0)) {
-    hipLaunchKernelGGL(k_uf_union, dim3(L.blocks_op), dim3(256), 0, st, B);
-  } else if (L.link_cap > 1) {
+  if (L.link_cap <= 1 || B.ntiles == 0) {
+    if (B.any_extra) hipLaunchKernelGGL(k_uf_union<true>, dim3(L.blocks_op), dim3(256), 0, st, B);
+    else hipLaunchKernelGGL(k_uf_union<false>, dim3(L.blocks_op), dim3(256), 0, st, B);
+  } else {
     hipLaunchKernelGGL(k_tile_union, dim3(B.ntiles), dim3(B.tile_cap > 4096 ? 1024 : 256), B.tile_cap * sizeof(int), st, B);
     hipLaunchKernelGGL(k_tile_cross, dim3(B.ntiles), dim3(B.tile_cap > 4096 ? 1024 : 256), 0, st, B);
   }
