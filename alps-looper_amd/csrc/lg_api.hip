@@ -505,7 +505,7 @@ int Batch::allocate(bool dynamic) {
   // the estimator accumulates into zeroed accumulators; the collector
   // clears each root's after reading it
   LG_HIP(hipMemset(acc, 0, (size_t)node_cap * sizeof(ClusterAcc)));
-  scan_nparts = (cap_bonds + 2047) / 2048 + (cap_sites + 2047) / 2048;
+  scan_nparts = cap_bonds / SCAN_CHUNK_MIN + cap_sites / SCAN_CHUNK_MIN + 2;
   if ((rc = alloc(scan_status, scan_nparts))) return rc;
   if ((rc = alloc(scan_ctl, 2))) return rc;
   LG_HIP(hipMemset(scan_status, 0, scan_nparts * sizeof(unsigned long long)));

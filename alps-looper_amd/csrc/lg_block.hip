@@ -65,23 +65,6 @@ __device__ __forceinline__ int wave_scan(int v) {
   return dpp_add<0x143, 0xc>(v);
 }
 
-// sum of v over the wave, in its last lane
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
-  return v + __longlong_as_double((long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo));
-}
-__device__ __forceinline__ double wave_total(double v) {
-  v = dpp_add<0x111, 0xf>(v);
-  v = dpp_add<0x112, 0xf>(v);
-  v = dpp_add<0x114, 0xf>(v);
-  v = dpp_add<0x118, 0xf>(v);
-  v = dpp_add<0x142, 0xa>(v);
-  return dpp_add<0x143, 0xc>(v);
-}
-
 // exclusive prefix of v over the workgroup's threads, and the total; wsum: 16
 // words, not those of the call before (one barrier between two uses is enough)
 __device__ __forceinline__ int blk_scan(int v, int* wsum, int* total) {

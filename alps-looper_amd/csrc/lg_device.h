@@ -29,6 +29,27 @@ __device__ __forceinline__ double wave_sum_d(double v) {
   return v;
 }
 
+// Sum of v over the wave, in its last lane, by DPP adds: the same sum by
+// shuffles is a dozen LDS operations, which for the collector's 19 terms took
+// a seventh of its time (chain L=1024, beta=1000: 30 -> 26 us).  k_estimate,
+// which has two and no register left, is faster with wave_sum_d (121 us
+// against 129 at square 128^2, beta=128).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
+  return v + __longlong_as_double((long long)(((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+__device__ __forceinline__ double wave_total(double v) {
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  return dpp_add<0x143, 0xc>(v);
+}
+
 // one of eight values by a run-time index, chosen from registers
 template <typename T>
 __device__ __forceinline__ T pick8(int i, T a0, T a1, T a2, T a3, T a4, T a5, T a6, T a7) {

@@ -55,7 +55,7 @@ struct DevBatch {
   ClusterAcc* acc;             // [nodes] (roots only)
   unsigned long long* scan_status;  // per scan chunk: epoch | state | value
   int* scan_ctl;                    // [0] chunk ticket, [1] launch epoch
-  double* col_part;            // [col_chunks(node_cap)][16] collector partial sums
+  double* col_part;            // [collector terms][chunks] collector partial sums, the chunks of the sweep's segments consecutive
   int* totals;                 // [0] operators, [1] nodes of the new configuration
   int* flags;
   uint32_t* sweep;             // [nchains]
@@ -89,7 +89,7 @@ struct DevBatch {
   int* sse_new;                // operator strings being built
   int* sse_perm;               // [ops] string position -> operator index of the new configuration
   int pairs;                   // every bond joins sites of opposite gauge factors (every L is even): pairs of segments apart
-  double* pair_part;           // [col_chunks(node_cap)][PAIR_COLS] sums over the chunk's pairs
+  double* pair_part;           // [PAIR_COLS][chunks] sums over the chunks' pairs
   int cross_parts;             // parts of 32 operators of a bond
   int ntiles, tile_cap;        // tiles of sites (ChainDev::tile0 ..) and segments that fit a tile's LDS
   const int* blk_nops;         // [nchains] operators per chain when each stands in its own region (else null)
@@ -111,6 +111,7 @@ struct BlockArgs {
 };
 
 constexpr int PAIR_COLS = 3;
+constexpr int SCAN_CHUNK_MIN = 256;  // bonds or sites of a status word of the scan, at least
 constexpr int TILE_CAP_MAX = 36864;  // segments (144 KB of LDS, the tables aside)
 // dynamic LDS beyond 64 KB for the tile kernel; false where the device has none
 bool tile_prepare();
@@ -145,7 +146,6 @@ void launch_cluster_stage(const DevBatch& B, const LaunchCfg& L, hipStream_t st,
 void launch_site_scan(const DevBatch& B, hipStream_t st);
 void launch_canon(const DevBatch& B, int chain, int nelem, int* canon, int* labels, int* roots,
                   hipStream_t st);
-int scan_blocks(const DevBatch& B);
 // the series walk of SSE chains, its string into bond-major operators, and
 // the flipped types back into the string (lg_sse.hip)
 void launch_sse_walk(const DevBatch& B, hipStream_t st);

@@ -395,9 +395,7 @@ k_diag_count_extra(DevBatch B) {
 // ---------------------------------------------------------------------------
 // scans: bond operator offsets and site segment offsets
 // ---------------------------------------------------------------------------
-constexpr int SCAN_ITEMS = 8;
-constexpr int SCAN_THREADS = 256;
-constexpr int SCAN_CHUNK = SCAN_ITEMS * SCAN_THREADS;
+constexpr int SCAN_THREADS = SCAN_CHUNK_MIN;
 
 __device__ __forceinline__ int site_events(const DevBatch& B, int gs) {
   const ChainDev& P = B.chains[B.site_chain[gs]];
@@ -459,22 +457,24 @@ __device__ int block_excl_scan(int v, int* total) {
 // the ticket before the scan), so the status words never need clearing.
 __global__ void k_scan_reset(DevBatch B) { scan_advance_epoch(B); }
 
+template <int ITEMS>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan(DevBatch B) {
+  constexpr int CHUNK = ITEMS * SCAN_THREADS;
   if (overflowed(B)) return;
   __shared__ int s_ticket, s_excl;
   if (threadIdx.x == 0) s_ticket = atomicAdd(B.scan_ctl, 1);
   __syncthreads();
   const int t = s_ticket;
   const uint32_t epoch = (uint32_t)B.scan_ctl[1];
-  const int nbB = (B.nbonds + SCAN_CHUNK - 1) / SCAN_CHUNK;
+  const int nbB = (B.nbonds + CHUNK - 1) / CHUNK;
   int blk = t, which = 0, n = B.nbonds, first = 0;
   if (blk >= nbB) { blk -= nbB; which = 1; n = B.nsites; first = nbB; }
-  const int base = blk * SCAN_CHUNK + threadIdx.x * SCAN_ITEMS;
-  int vals[SCAN_ITEMS];
-  bool empty[SCAN_ITEMS];
+  const int base = blk * CHUNK + threadIdx.x * ITEMS;
+  int vals[ITEMS];
+  bool empty[ITEMS];
   int sum = 0;
 #pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; ++k) {
+  for (int k = 0; k < ITEMS; ++k) {
     int v = 0;
     empty[k] = false;
     if (base + k < n) {
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan(DevBatch B) {
   int off = loc + s_excl;
   int* out = which ? B.soff_new : B.bo_new;
 #pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; ++k) {
+  for (int k = 0; k < ITEMS; ++k) {
     int i = base + k;
     if (i < n) {
       out[i] = off;
@@ -551,7 +551,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan(DevBatch B) {
     }
     off += vals[k];
   }
-  if (blk == (n - 1) / SCAN_CHUNK && threadIdx.x == 0) {
+  if (blk == (n - 1) / CHUNK && threadIdx.x == 0) {
     const int total = s_excl + tot;
     B.totals[which] = total;
     out[n] = total;
@@ -1708,7 +1708,7 @@ __global__ void __launch_bounds__(EST_THREADS) __attribute__((amdgpu_waves_per_e
       }
       __syncthreads();
       if (last && B.pairs && tid < PAIR_COLS) {
-        B.pair_part[(size_t)chunk * PAIR_COLS + tid] = hpair[tid];
+        B.pair_part[(size_t)tid * nchunks + chunk] = hpair[tid];
         hpair[tid] = 0;
       }
       for (int s = tid; s < HT; s += EST_THREADS) {
@@ -1782,7 +1782,7 @@ __global__ void __launch_bounds__(256) k_field_apply(DevBatch B) {
 // (susceptibility.h:177-198, stiffness.h:117-121) over the roots.
 // Collection is chunked: chunk j covers nodes [j*C, (j+1)*C), C = 256 *
 // chunk_items(M), and belongs to the chain of its first node; its sum over the roots of that
-// chain is written to col_part[j] (no atomics, fixed order), roots of other
+// chain is written to column j of col_part (no atomics, fixed order), roots of other
 // chains in the chunk (chunks straddling a chain boundary) are added to
 // rec_acc atomically.  end_sweep adds the partials of each chain in order.
 // An operator flips iff the clusters of its source-side legs l0 and u0 flip
@@ -1901,14 +1901,14 @@ __global__ void __launch_bounds__(COL_THREADS) k_flip_collect(DevBatch B, int cl
     if (cmax >= 0) {  // some lane of the wave holds a sum
       if (cmin == cmax) {
 #pragma unroll
-        for (int q = 0; q < NCOL; ++q) w[q] = wave_sum_d(w[q]);
-        if (lane_id() == 0) flush(cmax);
+        for (int q = 0; q < NCOL; ++q) w[q] = wave_total(w[q]);
+        if (lane_id() == 63) flush(cmax);
       } else if (cl >= 0) {
         flush(cl);
       }
     }
     __syncthreads();
-    if (threadIdx.x < NCOL) B.col_part[(size_t)chunk * NCOL + threadIdx.x] = slot[0][threadIdx.x];
+    if (threadIdx.x < NCOL) B.col_part[(size_t)threadIdx.x * nchunks + chunk] = slot[0][threadIdx.x];
     for (int s = NCOL + threadIdx.x; s < CSLOTS * NCOL; s += COL_THREADS) {
       const int k = s / NCOL, q = s % NCOL;
       const double val = slot[k][q];
@@ -1922,7 +1922,9 @@ __global__ void __launch_bounds__(COL_THREADS) k_flip_collect(DevBatch B, int cl
 // ---------------------------------------------------------------------------
 // end of sweep, one block per chain: add the chain's collector partials in a
 // fixed order, finish and store the record, advance the sweep counter.  The
-// last block to finish advances the record ring.
+// last block to finish advances the record ring.  A term's partials lie side by
+// side, so that a wave's load takes a few lines (chunk by chunk, 152 bytes
+// apart, and with sums by shuffles: 7.8 us at chain L=128, beta=100, now 6.0).
 // ---------------------------------------------------------------------------
 constexpr int END_THREADS = 256;
 
@@ -1951,22 +1953,23 @@ __global__ void __launch_bounds__(END_THREADS) k_end_sweep(DevBatch B) {
   for (int q = 0; q < NCOL; ++q) v[q] = 0;
   if (!bad) {
     const int start = B.soff_new[P.site_base], end = B.soff_new[P.site_base + P.N];
-    const int cchunk = chunk_items(B.totals[1]) * 256;  // as in k_flip_collect
+    const int M = B.totals[1], cchunk = chunk_items(M) * 256, nchunks = (M + cchunk - 1) / cchunk;  // as in k_flip_collect
     const int j0 = (start + cchunk - 1) / cchunk, j1 = (end + cchunk - 1) / cchunk;
+#pragma unroll 4
     for (int j = j0 + tid; j < j1; j += END_THREADS)
-      for (int q = 0; q < NCOL; ++q) v[q] += B.col_part[(size_t)j * NCOL + q];
+      for (int q = 0; q < NCOL; ++q) v[q] += B.col_part[(size_t)q * nchunks + j];
     if (B.pairs)  // the estimator's pairs, by the same chunks: clusters, usize^2 and smag^2, smag
       for (int j = j0 + tid; j < j1; j += END_THREADS) {
-        const double* p = B.pair_part + (size_t)j * PAIR_COLS;
-        v[0] += p[0];
-        v[6] += p[1];
-        v[14] += p[1];
-        v[17] += p[2];
+        const double t2 = B.pair_part[(size_t)nchunks + j];
+        v[0] += B.pair_part[j];
+        v[6] += t2;
+        v[14] += t2;
+        v[17] += B.pair_part[(size_t)2 * nchunks + j];
       }
   }
 #pragma unroll
-  for (int q = 0; q < NCOL; ++q) v[q] = wave_sum_d(v[q]);
-  if (lane_id() == 0)
+  for (int q = 0; q < NCOL; ++q) v[q] = wave_total(v[q]);
+  if (lane_id() == 63)
     for (int q = 0; q < NCOL; ++q) red[tid >> 6][q] = v[q];
   __syncthreads();
   double* rec = B.rec_acc + (size_t)c * R_COUNT;
@@ -2015,8 +2018,8 @@ __global__ void __launch_bounds__(END_THREADS) k_end_sweep(DevBatch B) {
       W->site_scale = candidate_scale(beta, P.site_w);
       W->dscale = candidate_scale(beta, P.dwsum);
     }
-    __threadfence();
-    is_last = (atomicAdd(B.end_count, 1) == (int)gridDim.x - 1);
+    // (a count alone: every block has read its slot before it adds)
+    is_last = gridDim.x == 1 || atomicAdd(B.end_count, 1) == (int)gridDim.x - 1;
   }
   __syncthreads();
   if (is_last && tid == 0) {
@@ -2134,8 +2137,20 @@ static void diag_dispatch(const DevBatch& B, const LaunchCfg& L, hipStream_t st,
 
 int col_chunks(int node_cap) { return (node_cap + COL_MIN_CHUNK - 1) / COL_MIN_CHUNK; }
 
-int scan_blocks(const DevBatch& B) {
-  return (B.nbonds + SCAN_CHUNK - 1) / SCAN_CHUNK + (B.nsites + SCAN_CHUNK - 1) / SCAN_CHUNK;
+// Items per thread: a thread's sites are a chain of loads each, and few chunks
+// leave the chip idle; many chunks lengthen the look-back (us with 1, 2, 4 and
+// 8 items: 4096 bonds and sites 5.4, 6.6, 8.9, 13.9; 49152: 8.6, 7.6, 9.9,
+// 15.6; 196608: 18.6, 13.8, 12.7, 18.4).
+static void launch_scan(const DevBatch& B, hipStream_t st) {
+  const int n = B.nbonds + B.nsites;
+  auto go = [&](auto kernel, int items) {
+    const int chunk = items * SCAN_THREADS;
+    hipLaunchKernelGGL(kernel, dim3((B.nbonds + chunk - 1) / chunk + (B.nsites + chunk - 1) / chunk), dim3(SCAN_THREADS), 0, st, B);
+  };
+  if (n <= 16384) go(k_scan<1>, 1);
+  else if (n <= 65536) go(k_scan<2>, 2);
+  else if (n <= 262144) go(k_scan<4>, 4);
+  else go(k_scan<8>, 8);
 }
 
 const char* const kKernelNames[NUM_PROFILED] = {
@@ -2179,7 +2194,7 @@ static void launch_sweep_sse(const DevBatch& B, const LaunchCfg& L, hipStream_t 
   mark(ev, 0, st);
   launch_sse_walk(B, st);  // also the scan's epoch
   mark(ev, 1, st);
-  hipLaunchKernelGGL(k_scan, dim3(scan_blocks(B)), dim3(SCAN_THREADS), 0, st, B);
+  launch_scan(B, st);
   mark(ev, 2, st);
   launch_sse_scatter(B, st);
   mark(ev, 3, st);
@@ -2192,11 +2207,10 @@ void launch_sweep(const DevBatch& B, const LaunchCfg& L, hipStream_t st, hipEven
     launch_sweep_sse(B, L, st, ev);
     return;
   }
-  const int sb = scan_blocks(B);
   mark(ev, 0, st);
   diag_dispatch(B, L, st, false);  // also clears the scan's ticket, next epoch
   mark(ev, 1, st);
-  hipLaunchKernelGGL(k_scan, dim3(sb), dim3(SCAN_THREADS), 0, st, B);
+  launch_scan(B, st);
   mark(ev, 2, st);
   diag_dispatch(B, L, st, true);
   mark(ev, 3, st);
@@ -2266,9 +2280,8 @@ void launch_exchange(const DevBatch& B, hipStream_t st) {
 }
 
 void launch_site_scan(const DevBatch& B, hipStream_t st) {
-  const int sb = scan_blocks(B);
   hipLaunchKernelGGL(k_scan_reset, dim3(1), dim3(1), 0, st, B);
-  hipLaunchKernelGGL(k_scan, dim3(sb), dim3(SCAN_THREADS), 0, st, B);
+  launch_scan(B, st);
 }
 
 void launch_canon(const DevBatch& B, int chain, int nelem, int* canon, int* labels, int* roots,

@@ -30,7 +30,7 @@ constexpr long long NA_OPS = LG_NOALLOC_MAX_OPS;
 constexpr long long NA_NODES = 2 * NA_OPS + NA_SITES;   // segments: max(events, 1) per site
 constexpr long long NA_ELEMS = NA_SITES + 4 * NA_OPS;   // label elements
 constexpr int NA_RING = 16;                             // record ring (one sweep is used)
-constexpr long long NA_SCAN = (NA_BONDS + 2047) / 2048 + (NA_SITES + 2047) / 2048;
+constexpr long long NA_SCAN = NA_BONDS / SCAN_CHUNK_MIN + NA_SITES / SCAN_CHUNK_MIN + 2;
 constexpr long long NA_COL = (NA_NODES + 1023) / 1024;  // collector chunks of at least 1024 nodes
 constexpr int FLAG_INPUT = 1 << 16;                     // invalid configuration (set by k_na_prep)
 
