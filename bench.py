@@ -202,12 +202,12 @@ def cpu_pool_baseline(chains, seconds, what, untimed=8, max_sweeps=64, sse=False
 
 def device_kernels(kernel, link):
     """device kernels behind a profiled sweep stage under linking setting
-    `link` (0: k_node_init + k_link_ops, which also unites; 1: k_link_site;
-    else the LDS-staged k_link), by their short names"""
+    `link` (0: k_link_ops; 1: k_link_site; else the LDS-staged k_link, after
+    which large chains unite by tiles), by their short names"""
     if kernel == "link":
-        return ("node_init", "link_ops") if link == 0 else ("link_site",) if link == 1 else ("link",)
+        return ("link_ops",) if link == 0 else ("link_site",) if link == 1 else ("link",)
     if kernel == "uf_union":
-        return () if link == 0 else ("uf_union",)
+        return ("uf_union",) if link <= 1 else ("uf_union", "tile_union", "tile_cross")
     return (kernel,)
 
 
@@ -220,7 +220,7 @@ def measured_traffic(name, kernel, nop_mean, link=0):
     try:
         with open(path) as f:
             d = json.load(f)
-        ks = device_kernels(kernel, link)
+        ks = [k for k in device_kernels(kernel, link) if k in d["kernels"]]
         return sum(d["kernels"][k]["bytes_per_op"] for k in ks) * nop_mean if ks else None
     except (OSError, KeyError, TypeError):
         return None
@@ -228,15 +228,11 @@ def measured_traffic(name, kernel, nop_mean, link=0):
 
 def kernel_bytes(compress, link=0):
     """algorithmic bytes per operator of each kernel: without the compress
-    pass the estimator's own walk does the compression; the per-operator
-    linking kernel (link 0) also does the unions"""
+    pass the estimator's own walk does the compression"""
     b = dict(BYTES_PER_OP)
     if not compress:
         b["estimate"] += b["uf_compress"]
         b["uf_compress"] = 0.0
-    if link == 0:
-        b["link"] += b["uf_union"]
-        b["uf_union"] = 0.0
     b["chain_sweep"] = sum(BYTES_PER_OP.values())  # one workgroup per chain: the whole sweep
     return b
 
