@@ -208,6 +208,8 @@ def device_kernels(kernel, link):
         return ("link_ops",) if link == 0 else ("link_site",) if link == 1 else ("link",)
     if kernel == "uf_union":
         return ("uf_union",) if link <= 1 else ("uf_union", "tile_union", "tile_cross")
+    if kernel == "chain_sweep":
+        return ("chain_sweeps",)
     return (kernel,)
 
 
