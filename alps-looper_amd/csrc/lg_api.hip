@@ -251,8 +251,12 @@ static double expected_ops(const lg_params& p, const ChainDev& d) {
 // kernels.  Fitted to chains of 41 to 24000 operators on 16 to 3072 bonds
 // (one workgroup: 18 us at 41 operators, 22 at 450, 65 at 3000 on 512 bonds,
 // 40 at 350 on 2048, 540 at 24000 on 2048, where the clusters' accumulators
-// take several passes) and on the flat kernels' launches (65 us at 450
-// operators, 83 at 8900, 140 with virtual sites, 1050 at 3.2M in 512 chains).
+// take several passes) and on the flat kernels' launches (60 us at 900
+// operators, 73 at 8900, 131 with virtual sites, 1030 at 3.2M in 512 chains).
+// Near the line, one workgroup and the launches: chain L=64, beta=70 69 and 76
+// us; square 32^2, beta=2.5 67 and 68; S=1 chain L=64, beta=30 111 and 145;
+// square 24^2 in a transverse field, beta=6 92 and 93; 32 chains of 16^2,
+// beta=16 104 and 127.
 static double block_us(double n, int bonds) {
   return 14.0 + 0.016 * n + 0.012 * bonds + 0.01 * std::max(0.0, n - 12000.0);
 }
