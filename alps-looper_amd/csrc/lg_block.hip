@@ -615,8 +615,8 @@ __device__ __forceinline__ void seg_winding(int fl, int flo, int& d0, int& d1) {
 // (1024 threads: 128 VGPRs; one workgroup per CU at the full LDS)
 template <bool GEN>
 __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) {
-  if (overflowed(B)) return;
   __shared__ int s_next, s_ncand, s_wsum[2][16];
+  if (block_overflowed(B, &s_ncand)) return;
   __shared__ double s_red[16][NCOL];
   int* const ws0 = s_wsum[0];
   int* const ws1 = s_wsum[1];

@@ -460,11 +460,13 @@ __global__ void k_scan_reset(DevBatch B) { scan_advance_epoch(B); }
 template <int ITEMS>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan(DevBatch B) {
   constexpr int CHUNK = ITEMS * SCAN_THREADS;
-  if (overflowed(B)) return;
   __shared__ int s_ticket, s_excl;
-  if (threadIdx.x == 0) s_ticket = atomicAdd(B.scan_ctl, 1);
+  // (one thread decides for the workgroup, as in block_overflowed: the last
+  // bond chunk may set the flag while a site chunk starts)
+  if (threadIdx.x == 0) s_ticket = overflowed(B) ? -1 : atomicAdd(B.scan_ctl, 1);
   __syncthreads();
   const int t = s_ticket;
+  if (t < 0) return;
   const uint32_t epoch = (uint32_t)B.scan_ctl[1];
   const int nbB = (B.nbonds + CHUNK - 1) / CHUNK;
   int blk = t, which = 0, n = B.nbonds, first = 0;

@@ -53,7 +53,7 @@ __device__ __forceinline__ int with_lane(int v, int l, int x) { return lane_id()
 // operator stored in the loop 8.9 ms.
 __global__ void __launch_bounds__(SSE_THREADS) k_sse_walk(DevBatch B) {
   if (blockIdx.x == 0 && threadIdx.x == 0) scan_advance_epoch(B);  // for k_scan, which follows
-  if (overflowed(B)) return;
+  if (__builtin_amdgcn_readfirstlane((int)overflowed(B))) return;  // (another chain may set it meanwhile: one answer a wave)
   const int c = blockIdx.x;
   const ChainDev& P = B.chains[c];
   __shared__ uint32_t spw[SSE_MAX_SITES / 32];            // spins, a bit each
