@@ -788,8 +788,12 @@ void Batch::choose_block() {
   std::vector<int> idx(nc);
   for (size_t i = 0; i < nc; ++i) idx[i] = order[i].second;
   // its buffers, once (the order, and k_pack's bases; counts; segment scratch)
-  if (!blk_info && (alloc(blk_order, 3 * (size_t)cap_chains) || alloc(blk_nops, cap_chains) || alloc(blk_nnodes, cap_chains) ||
+  const bool fresh = !blk_info;
+  if (fresh && (alloc(blk_order, 3 * (size_t)cap_chains) || alloc(blk_nops, cap_chains) || alloc(blk_nnodes, cap_chains) ||
                      alloc(blk_root, node_cap) || alloc(blk_len, node_cap) || alloc(blk_info, node_cap)))
+    return;
+  if (fresh && (hipMemset(blk_nops, 0, cap_chains * sizeof(int)) != hipSuccess ||
+                hipMemset(blk_nnodes, 0, cap_chains * sizeof(int)) != hipSuccess))
     return;
   if (hipMemcpy(blk_order, idx.data(), nc * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) return;
   blk_fit = true;
@@ -835,6 +839,7 @@ int Batch::run_block(uint32_t n, uint32_t slot0) {
 
 int Batch::ensure_packed() {
   if (!blk_regions) return LG_OK;
+  if (int rc = config_error()) return rc;  // (the counts of an overflowed sweep are not its arrays')
   const size_t nc = chains.size();
   std::vector<int> n(nc), m(nc), base(2 * nc);
   LG_HIP(hipStreamSynchronize(stream));
@@ -1043,7 +1048,9 @@ int Batch::flags_error() const {
 }
 
 int Batch::check_flags() {
-  LG_HIP(hipMemcpy(&flags_seen, flags, sizeof(int), hipMemcpyDeviceToHost));
+  int f = 0;
+  LG_HIP(hipMemcpy(&f, flags, sizeof(int), hipMemcpyDeviceToHost));
+  see_flags(f);
   return flags_error();
 }
 
@@ -1095,7 +1102,9 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
     const size_t words = out ? (size_t)chunk * nc * R_COUNT : 0;
     LG_HIP(hipMemcpyAsync(rec_host, flags, (REC_HEAD + words) * sizeof(double), hipMemcpyDeviceToHost, stream));
     LG_HIP(hipStreamSynchronize(stream));
-    std::memcpy(&flags_seen, rec_host, sizeof(int));
+    int f;
+    std::memcpy(&f, rec_host, sizeof(int));
+    see_flags(f);
     if ((rc = flags_error())) return rc;
     if (out) {
       static_assert(sizeof(lg_sweep_record) == R_COUNT * sizeof(double), "record layout");
@@ -1390,6 +1399,7 @@ int Batch::set_config(int c, const int32_t* spins_in, const int32_t* bond_offset
   uint32_t sw = (uint32_t)sweep;
   LG_HIP(hipMemcpy(d_sweep, &sw, sizeof(uint32_t), hipMemcpyHostToDevice));
   host_sweep[c] = sweep;
+  config_lost = false;
   return sync_schedule();
 }
 
@@ -1415,6 +1425,7 @@ __global__ void __launch_bounds__(256) k_export(const uint8_t* spins, const int*
 
 int Batch::get_config(int c, int32_t* spins, int32_t* bond_offsets, double* times, int32_t* types) {
   if (chains.size() != 1) return set_error(LG_ERR_UNSUPPORTED, "get_config needs a single-chain handle");
+  if (int rc = config_error()) return rc;
   const ChainDev& d = chains[c];
   const State& s = st[cur];
   const bool ops = times || types;
@@ -1456,6 +1467,7 @@ int Batch::get_config(int c, int32_t* spins, int32_t* bond_offsets, double* time
 }
 
 int Batch::num_ops(int c, long long* n) {
+  if (int rc = config_error()) return rc;
   if ((size_t)c < known_ops.size()) {
     *n = known_ops[c];
     return LG_OK;
@@ -1480,6 +1492,7 @@ int Batch::chain_config(int c, std::vector<int>& spins, std::vector<int>& bo, st
   if (!swept_since_layout && (chains[c].old_site_base != chains[c].site_base ||
                               chains[c].old_bond_base != chains[c].bond_base))
     return set_error(LG_ERR_STATE, "chain moved since its last sweep");
+  if (int rc = config_error()) return rc;
   if (int rc = ensure_packed()) return rc;
   LG_HIP(hipStreamSynchronize(stream));
   const ChainDev& d = chains[c];
@@ -1564,6 +1577,7 @@ int Batch::load_configs(const std::vector<HostConfig>& cfg) {
   old_ext_sites = nsites;
   old_ext_bonds = nbonds;
   old_ext_nodes = node_base;
+  config_lost = false;
   return sync_schedule();
 }
 

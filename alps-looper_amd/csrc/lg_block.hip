@@ -763,8 +763,10 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
     __syncthreads();
     const int m = uni(blk_prefix(S.sn, N, ws0));
     if (n > P.blk_opcap || m > P.blk_nodecap) {
-      // the operators or segments do not fit (uniform over the workgroup):
-      // the configuration before this sweep stays
+      // the operators or segments do not fit (uniform over the workgroup).
+      // The offsets of the launch's earlier sweeps are not written out and
+      // the host takes the next arrays for the configuration: none is whole
+      // from here on, and the host gives none out (Batch::config_lost)
       if (tid == 0) atomicOr(B.flags, n > P.blk_opcap ? FLAG_OP_OVERFLOW : FLAG_NODE_OVERFLOW);
       return;
     }

@@ -150,6 +150,8 @@ class Batch {
   int capture(int from);
   int check_flags();
   int flags_error() const;
+  void see_flags(int f) { flags_seen = f; config_lost = config_lost || f != 0; }
+  int config_error() const { return config_lost ? flags_error() : LG_OK; }
   void choose_tiles();
   void choose_block();
   int run_block(uint32_t n, uint32_t slot0);
@@ -196,6 +198,7 @@ class Batch {
   unsigned char* cfg_host = nullptr;              // pinned memory for a configuration on its way out
   static constexpr size_t CFG_HOST_BYTES = 256 << 10;
   int flags_seen = 0;                             // the error flags as last read
+  bool config_lost = false;                       // a sweep overflowed: neither state holds a whole configuration
   std::vector<long long> known_ops;               // operators per chain, while the last records tell them
   int* ring_pos = nullptr;
   int* end_count = nullptr;

@@ -131,7 +131,10 @@ int lg_chain_info(lg_chain* h, int32_t* n_sites, int32_t* n_bonds, int64_t* n_op
 /* configuration (checkpoint content of path_integral.C:111-124): spins at
  * tau=0 [n_sites] (0 = up), operators in bond-major order with bond offsets
  * [n_bonds+1], times [n_ops] and type (offdiagonal | graph << 2, operator.h
- * layout) [n_ops]. */
+ * layout) [n_ops].  A sweep that ended with LG_ERR_CAPACITY leaves no whole
+ * configuration: this call, lg_chain_info's and lg_batch_chain_info's n_ops,
+ * lg_chain_save and lg_batch_add return the same error until a configuration
+ * is set or loaded (the handle sweeps no more). */
 int lg_chain_get_config(lg_chain* h, int32_t* spins, int32_t* bond_offsets, double* times,
                         int32_t* types);
 int lg_chain_set_config(lg_chain* h, const int32_t* spins, const int32_t* bond_offsets,

@@ -55,3 +55,25 @@ def test_error_and_the_handles_after_it(loopgpu, flat, sweeps):
     a, b = loopgpu.Chain(p), loopgpu.Chain(p)
     b.set_launch(group=8)
     assert np.array_equal(a.sweep(3)[:, :2], b.sweep(3)[:, :2])
+
+
+@pytest.mark.parametrize("flat", [False, True])
+@pytest.mark.parametrize("sweeps", [1, 2, 5])
+def test_no_configuration_is_given_out(loopgpu, flat, sweeps):
+    """neither state's arrays hold a whole configuration then; one that is set
+    comes back as it was"""
+    c = _overflow(loopgpu, flat, sweeps)
+    for call in (c.info, c.get_config, c.save, lambda: c.set_schedule([1, 9], [0.1, 0.25])):
+        with pytest.raises(loopgpu.LoopGPUError) as e:
+            call()
+        assert e.value.code == CAPACITY
+    d = loopgpu.Chain(loopgpu.params(loopgpu.CHAIN, 16, 4.0, 1.0, 1.0, seed=4))
+    d.sweep(9)
+    ref = d.get_config()
+    c.set_config(*ref, 9)
+    for x, y in zip(c.get_config(), ref):
+        assert np.array_equal(x, y)
+    assert c.info() == d.info()
+    with pytest.raises(loopgpu.LoopGPUError) as e:
+        c.sweep(1)
+    assert e.value.code == CAPACITY
