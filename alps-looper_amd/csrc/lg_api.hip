@@ -854,6 +854,7 @@ int Batch::ensure_packed() {
   }
   int* const d_base = blk_order + cap_chains;
   LG_HIP(hipMemcpy(d_base, base.data(), 2 * nc * sizeof(int), hipMemcpyHostToDevice));
+  drop_stale_error();
   launch_pack(dev(cur), blk_nops, blk_nnodes, d_base, d_base + nc, stream);
   LG_HIP(hipGetLastError());
   LG_HIP(hipStreamSynchronize(stream));
@@ -1083,6 +1084,7 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
   if (rc) return rc;
   const size_t nc = chains.size();
   if (nc == 0 || n == 0) return LG_OK;
+  drop_stale_error();
   known_ops.clear();
   const bool block = block_form();
   if (!block && (rc = ensure_packed())) return rc;
@@ -1226,6 +1228,7 @@ int Batch::profile(uint32_t n, double* ms) {
   if (rc) return rc;
   const int K = NUM_SWEEP_KERNELS;
   for (int i = 0; i < NUM_PROFILED; ++i) ms[i] = 0;
+  drop_stale_error();
   known_ops.clear();
   if (block_form()) {  // one workgroup per chain: the launches as a whole
     hipEvent_t e0, e1;
@@ -1439,6 +1442,7 @@ int Batch::get_config(int c, int32_t* spins, int32_t* bond_offsets, double* time
       int32_t* const hs = hy + n;
       int32_t* const hb = hs + d.N;
       const int blocks = (int)std::min<size_t>(64, (n + d.N + d.Nb + 256) / 256);
+      drop_stale_error();
       hipLaunchKernelGGL(k_export, dim3(blocks), dim3(256), 0, stream, s.spins, s.bo, s.ot, s.oi, d.N, d.Nb, (int)n,
                          spins ? hs : nullptr, bond_offsets ? hb : nullptr, times ? ht : nullptr, types ? hy : nullptr);
       LG_HIP(hipGetLastError());
@@ -1725,6 +1729,7 @@ int Batch::cluster_only(const int32_t* spins_in, const int32_t* bond_offsets, co
   LG_HIP(hipMemcpy(d_sweep, &sw, sizeof(uint32_t), hipMemcpyHostToDevice));
   LG_HIP(hipMemset(ring_pos, 0, sizeof(int)));
   DevBatch B = dev(from);
+  drop_stale_error();
   launch_site_scan(B, stream);
   launch_cluster_stage(B, cfg, stream);
   LG_HIP(hipGetLastError());

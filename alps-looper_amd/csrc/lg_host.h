@@ -42,6 +42,11 @@ struct Capacity {
   long long sites = 0, bonds = 0, ops = 0, cand = 0;
 };
 
+// The runtime keeps a thread's last error until it is asked for: what an
+// earlier call left (an allocation that failed, another library's call) would
+// come out of the check after this call's launches.
+inline void drop_stale_error() { (void)hipGetLastError(); }
+
 class Batch {
  public:
   ~Batch();

@@ -279,6 +279,7 @@ int lg_cluster_config_noalloc(const lg_params* p, const int32_t* spins, const in
     hipError_t e_ = (call);                                                                 \
     if (e_ != hipSuccess) return set_error(LG_ERR_DEVICE, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
+  drop_stale_error();
   // descriptor, sweep index, and the control words that must start at zero
   // (scan ticket and epoch, totals, flags, ring position, end count; scan
   // status words; record accumulators)
