@@ -294,6 +294,7 @@ int Batch::alloc(T*& ptr, size_t n) {
 
 int Batch::init_for_config(const lg_params* p, long long nops) {
   min_op_cap = nops + 1024;
+  blk_barred = true;  // (the cluster stage alone)
   return init(p, 1);
 }
 
@@ -387,15 +388,20 @@ int Batch::init_exchange(const lg_params& p, const double* betas, int n, uint32_
     cap.cand += (long long)ds[t].Nb * cand_cap;
     ops_max = std::max(ops_max, f.ops);
   }
-  // one workgroup per chain keeps every chain in a region of its own, which
-  // has to hold the largest beta's operators
-  if (n * ops_max <= (1ll << 26)) {
-    blk_exchange_ops = ops_max;
-    cap.ops = std::max(cap.ops, n * ops_max);
-  }
-  if ((rc = reserve(cap, false))) return rc;
   params = ps;
   swap_betas = true;
+  // One workgroup per chain keeps every chain in a region of its own, which
+  // has to hold the largest beta's operators.  Room for that only where the
+  // batch then takes that form (32 replicas of 128^2 up to beta=32, which do
+  // not: 2.9 GB, with it 8.8).
+  device_limits();
+  if (n * ops_max <= (1ll << 26) && plan_block(ds, ops_max, n * ops_max, 2 * n * ops_max + cap.sites)) {
+    blk_exchange_ops = ops_max;
+    cap.ops = std::max(cap.ops, n * ops_max);
+  } else {
+    blk_barred = true;
+  }
+  if ((rc = reserve(cap, false))) return rc;
   if ((rc = set_layout(ds, std::vector<uint64_t>(n, 0)))) return rc;
   if ((rc = reset_state())) return rc;
   if ((rc = alloc(xslot, n)) || (rc = alloc(xbeta, n)) || (rc = alloc(xscale, n)) ||
@@ -412,7 +418,6 @@ int Batch::init_exchange(const lg_params& p, const double* betas, int n, uint32_
   LG_HIP(hipMemset(xacc, 0, (n - 1) * sizeof(unsigned long long)));
   LG_HIP(hipMemset(xstep, 0, sizeof(uint32_t)));
   nslots = n;
-  if (blk_exchange_ops == 0) blk_fit = false;
   xkey0 = seed;
   xkey1 = 0xffffffffu;
   invalidate_graphs();
@@ -468,11 +473,22 @@ int Batch::reserve(const Capacity& cap, bool dynamic) {
   node_cap = (int)ncap;
   cand_total = cap.cand;
   LG_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  return allocate(dynamic);
+  // server batches: their mixes hold jobs too large for one workgroup, and
+  // their sweeps replay the graph of each layout
+  blk_barred = blk_barred || dynamic;
+  return allocate();
 }
 
-int Batch::allocate(bool dynamic) {
+// what the device has for the choice of the sweep's form
+void Batch::device_limits() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) cus = n;
+  blk_lds_grant = !blk_barred && block_prepare() ? BLOCK_LDS_MAX : 0;
+}
+
+int Batch::allocate() {
   int rc = 0;
+  device_limits();
   for (int i = 0; i < 2; ++i) {
     State& s = st[i];
     if ((rc = alloc(s.spins, cap_sites))) return rc;
@@ -514,10 +530,7 @@ int Batch::allocate(bool dynamic) {
   if ((rc = alloc(scan_ctl, 2))) return rc;
   LG_HIP(hipMemset(scan_status, 0, scan_nparts * sizeof(unsigned long long)));
   LG_HIP(hipMemset(scan_ctl, 0, 2 * sizeof(int)));
-  // one workgroup per chain, except for server batches, whose mixes hold jobs
-  // too large for it and whose sweeps replay the graph of each layout
   if (!tile_prepare()) return set_error(LG_ERR_DEVICE, "the device refuses the tile kernel's LDS");
-  blk_lds_grant = !dynamic && block_prepare() ? BLOCK_LDS_MAX : 0;
   if ((rc = alloc(col_part, (size_t)col_chunks(node_cap) * NUM_COLLECTOR_TERMS))) return rc;
   if ((rc = alloc(pair_part, (size_t)col_chunks(node_cap) * PAIR_COLS))) return rc;
   if ((rc = alloc(totals, 2))) return rc;
@@ -550,10 +563,6 @@ int Batch::allocate(bool dynamic) {
   known_ops.clear();
   LG_HIP(hipMemset(ring_pos, 0, sizeof(int)));
   LG_HIP(hipMemset(totals, 0, 2 * sizeof(int)));
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
   cfg.blocks_op = std::max(64, cus * 8);
   cfg.blocks_node = std::max(64, cus * 8);
   return LG_OK;
@@ -739,26 +748,24 @@ most.push_back(2 * d.beta / d.N * (d.offset_total + d.nb_real * (std::fabs(p.jz)
     ntiles += set_tiles(chains[c], ntiles, swap_betas ? mean_max : mean[c], swap_betas ? most_max : most[c], target, tile_cap);
 }
 
-// Regions of the chains, and whether the batch takes one workgroup per chain.
-void Batch::choose_block() {
-  blk_fit = false;
-  const size_t nc = chains.size();
-  if (nc == 0 || is_sse() || blk_lds_grant <= 0) return;
+// Regions of the chains ds, of region operators each (0: what the chain by
+// itself may need), in arrays of op_room and node_room, and whether one
+// workgroup per chain is to sweep them.
+bool Batch::plan_block(std::vector<ChainDev>& ds, long long region, long long op_room, long long node_room) {
+  const size_t nc = ds.size();
+  if (nc == 0 || ds[0].sse || blk_lds_grant <= 0) return false;
   double most = 0, longest = 0, sum = 0, total = 0;
   long long ops = 0, nodes = 0;
   int lds = 0, least = 0;
   bool general = false;
-  std::vector<std::pair<double, int>> order(nc);
   for (size_t c = 0; c < nc; ++c) {
-    ChainDev& d = chains[c];
+    ChainDev& d = ds[c];
     // (site pairs in 16 + 16 bits, candidate ranks in 10, tables in LDS)
-    if (d.N > 0xffff || d.Nb > 16384 || d.cand_cap > 1024) return;
-    // operators of a chain's region: a replica of an exchange may come to the
-    // largest beta, one chain has the whole capacity
-    long long cap = nc == 1 ? op_cap : footprint(params[c]).ops;
-    if (blk_exchange_ops > 0) cap = blk_exchange_ops;
+    if (d.N > 0xffff || d.Nb > 16384 || d.cand_cap > 1024) return false;
+    // (one chain has the whole capacity)
+    const long long cap = region > 0 ? region : (nc == 1 ? op_room : footprint(params[c]).ops);
     const long long ncap = 2 * cap + d.N;
-    if (ops + cap > op_cap || nodes + ncap > node_cap) return;
+    if (ops + cap > op_room || nodes + ncap > node_room) return false;
     d.blk_op = (int)ops;
     d.blk_node = (int)nodes;
     d.blk_opcap = (int)cap;
@@ -766,8 +773,7 @@ void Batch::choose_block() {
     ops += cap;
     nodes += ncap;
     const double n = expected_ops(params[c], d);
-    if (n > 1.0e5) return;
-    order[c] = {n, (int)c};
+    if (n > 1.0e5) return false;
     most = std::max(most, n);
     const double us = block_us(n, d.Nb);
     longest = std::max(longest, us);
@@ -777,26 +783,39 @@ void Batch::choose_block() {
     lds = std::max(lds, block_lds_for(d, (int)(1.1 * n) + 64));
     general = general || d.nv > 1 || d.Nb > d.nb_lat;
   }
-  if (least > blk_lds_grant) return;
+  if (least > blk_lds_grant) return false;
   blk_lds = std::min(std::max(lds, least), blk_lds_grant);
   blk_threads = most <= 256 ? 256 : (most <= 1024 ? 512 : 1024);
   blk_general = general;
   // a batch lasts as long as its longest chain, or as its chains over the CUs
   blk_us = std::max(longest, sum / std::max(cus, 1));
-  if (blk_us > flat_us(total, general)) return;
-  std::sort(order.begin(), order.end(), [](const auto& x, const auto& y) { return x.first != y.first ? x.first > y.first : x.second < y.second; });
-  std::vector<int> idx(nc);
-  for (size_t i = 0; i < nc; ++i) idx[i] = order[i].second;
-  // its buffers, once (the order, and k_pack's bases; counts; segment scratch)
-  const bool fresh = !blk_info;
-  if (fresh && (alloc(blk_order, 3 * (size_t)cap_chains) || alloc(blk_nops, cap_chains) || alloc(blk_nnodes, cap_chains) ||
-                     alloc(blk_root, node_cap) || alloc(blk_len, node_cap) || alloc(blk_info, node_cap)))
-    return;
-  if (fresh && (hipMemset(blk_nops, 0, cap_chains * sizeof(int)) != hipSuccess ||
-                hipMemset(blk_nnodes, 0, cap_chains * sizeof(int)) != hipSuccess))
-    return;
-  if (hipMemcpy(blk_order, idx.data(), nc * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) return;
-  blk_fit = true;
+  return blk_us <= flat_us(total, general);
+}
+
+// A batch that plan_block accepts: the order of its workgroups (largest chains
+// first) and its buffers.
+void Batch::choose_block() {
+  blk_fit = false;
+  if (!plan_block(chains, blk_exchange_ops, op_cap, node_cap)) return;
+  const size_t nc = chains.size(), cc = cap_chains;
+  std::vector<std::pair<double, int>> order(nc);
+  for (size_t c = 0; c < nc; ++c) order[c] = {-expected_ops(params[c], chains[c]), (int)c};
+  std::sort(order.begin(), order.end());
+  // one allocation: segment scratch, then the order, k_pack's bases and the
+  // chains' counts (0: nothing has been swept yet)
+  if (!blk_len) {
+    unsigned char* mem = nullptr;
+    if (alloc(mem, (size_t)node_cap * 16 + 5 * cc * sizeof(int))) return;
+    blk_len = (double*)mem;
+    blk_root = (int*)(blk_len + node_cap);
+    blk_info = (uint32_t*)(blk_root + node_cap);
+    blk_order = (int*)(blk_info + node_cap);
+    blk_nops = blk_order + 3 * cc;
+    blk_nnodes = blk_nops + cc;
+  }
+  std::vector<int> head(5 * cc, 0);
+  for (size_t i = 0; i < nc; ++i) head[i] = order[i].second;
+  blk_fit = hipMemcpy(blk_order, head.data(), head.size() * sizeof(int), hipMemcpyHostToDevice) == hipSuccess;
 }
 
 // n sweeps with one workgroup per chain, records to the ring from slot0 on.

@@ -146,7 +146,8 @@ class Batch {
   // new bases (contiguous in the given order), chain tables, sweep counters;
   // check_old: also check the previous bases a relayout leaves the chains with
   int set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sweeps, bool check_old = false);
-  int allocate(bool dynamic);
+  int allocate();
+  void device_limits();
   int reset_state();
   void release();
   void invalidate_graphs();
@@ -158,6 +159,7 @@ class Batch {
   void see_flags(int f) { flags_seen = f; config_lost = config_lost || f != 0; }
   int config_error() const { return config_lost ? flags_error() : LG_OK; }
   void choose_tiles();
+  bool plan_block(std::vector<ChainDev>& ds, long long region, long long op_room, long long node_room);
   void choose_block();
   int run_block(uint32_t n, uint32_t slot0);
   // st[cur] in the packed form (the chains' operators and segments consecutive)
@@ -220,6 +222,7 @@ class Batch {
   // one workgroup per chain (lg_block.hip): every chain fits and it is the
   // faster form (blk_fit), unless launch settings were given (blk_off);
   // blk_regions: st[cur] stands in the chains' own regions
+  bool blk_barred = false;       // never one workgroup per chain
   bool blk_fit = false, blk_off = false, blk_regions = false, blk_general = false;
   bool swap_betas = false;       // replica exchange: a chain comes to every temperature
   int cross_parts = 1, ntiles = 0, tile_cap = 0;  // tiles of sites of the flat kernels' unions
