@@ -1146,11 +1146,12 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
 int Batch::tune(uint32_t sweeps_per_trial) {
   if (sweeps_per_trial == 0) sweeps_per_trial = 8;
   // the first trial warms state and code, and times one workgroup per chain
-  // (after its first sweep) where the batch can take it
+  // (after its first sweep) where the batch can take it; a trial of one sweep
+  // leaves nothing to time, and the rule's choice stands
   blk_off = false;
   int rc = run(1, nullptr);
   if (rc) return rc;
-  double block_t = blk_us * 1e-6;
+  double block_t = 0;
   if (sweeps_per_trial > 1) {
     const auto t0 = std::chrono::steady_clock::now();
     if ((rc = run(sweeps_per_trial - 1, nullptr))) return rc;
