@@ -79,3 +79,21 @@ def test_cold_batches(loopgpu, chains, kind, L, lo, hi, least, kw):
     assert most > least
     a.set_launch(group=8)
     _same(a.run(1), b.run(1))
+
+
+def test_pairs_of_many_chains_in_a_chunk(loopgpu):
+    """the flat estimator's chunk of 1024 to 4096 segments over chains of two
+    segments each up to a few hundred: more of them than it has slots, and
+    chunks that begin inside a chain"""
+    ps = [loopgpu.params(0, 2 + 2 * (i % 5), be, 1.0, 1.0, seed=5, chain_id=i) for i, be in enumerate(_betas(0.1, 20.0, 400))]
+    a, b, c = loopgpu.Batch(ps), loopgpu.Batch(ps), loopgpu.Batch(ps)
+    b.set_launch(group=8, link=0)
+    c.set_launch(group=8, link=512, compress=1)
+    assert _one_workgroup(a)
+    b.run(1, records=False)
+    c.run(1, records=False)
+    for n in (1, 30):
+        print("chains", n, flush=True)
+        x = a.run(n)
+        _same(x, b.run(n))
+        _same(x, c.run(n))
