@@ -804,12 +804,13 @@ void Batch::choose_block() {
   // one allocation: segment scratch, then the order, k_pack's bases and the
   // chains' counts (0: nothing has been swept yet)
   if (!blk_len) {
+    const size_t m = ((size_t)node_cap + 63) & ~(size_t)63;  // (whole lines)
     unsigned char* mem = nullptr;
-    if (alloc(mem, (size_t)node_cap * 16 + 5 * cc * sizeof(int))) return;
+    if (alloc(mem, m * 16 + 5 * cc * sizeof(int))) return;
     blk_len = (double*)mem;
-    blk_root = (int*)(blk_len + node_cap);
-    blk_info = (uint32_t*)(blk_root + node_cap);
-    blk_order = (int*)(blk_info + node_cap);
+    blk_root = (int*)(blk_len + m);
+    blk_info = (uint32_t*)(blk_root + m);
+    blk_order = (int*)(blk_info + m);
     blk_nops = blk_order + 3 * cc;
     blk_nnodes = blk_nops + cc;
   }
@@ -842,8 +843,10 @@ int Batch::run_block(uint32_t n, uint32_t slot0) {
     A.root_of = blk_root;
     A.seg_len = blk_len;
     A.seg_info = blk_info;
+    if (blk_unseen && nslots <= 1) launch_chain_stop(B, stream);
     launch_chain_sweeps(B, A, blk_general, blk_threads, stream);
-    if (nslots > 1) {
+    blk_unseen = true;
+    if (nslots > 1) {  // (passes the flags on as well)
       B.blk_nops = blk_nops;
       launch_exchange(B, stream);
     }
@@ -1068,8 +1071,8 @@ int Batch::flags_error() const {
 }
 
 int Batch::check_flags() {
-  int f = 0;
-  LG_HIP(hipMemcpy(&f, flags, sizeof(int), hipMemcpyDeviceToHost));
+  int f[2];
+  LG_HIP(hipMemcpy(f, flags, sizeof(f), hipMemcpyDeviceToHost));
   see_flags(f);
   return flags_error();
 }
@@ -1123,8 +1126,8 @@ int Batch::run(uint32_t n, lg_sweep_record* out) {
     const size_t words = out ? (size_t)chunk * nc * R_COUNT : 0;
     LG_HIP(hipMemcpyAsync(rec_host, flags, (REC_HEAD + words) * sizeof(double), hipMemcpyDeviceToHost, stream));
     LG_HIP(hipStreamSynchronize(stream));
-    int f;
-    std::memcpy(&f, rec_host, sizeof(int));
+    int f[2];
+    std::memcpy(f, rec_host, sizeof(f));
     see_flags(f);
     if ((rc = flags_error())) return rc;
     if (out) {

@@ -332,7 +332,7 @@ __device__ __forceinline__ void blk_draw(const DevBatch& B, const ChainDev& P, u
         list[at] = (double)T * TGRID_INV;
         list_bond[at] = (uint32_t)b | ((uint32_t)g << 14) | ((uint32_t)k << 16);
       } else {
-        atomicOr(B.flags, FLAG_CAND_OVERFLOW);
+        atomicOr(B.flags + 1, FLAG_CAND_OVERFLOW);
       }
     }
     if (G > 1) {
@@ -615,8 +615,10 @@ __device__ __forceinline__ void seg_winding(int fl, int flo, int& d0, int& d1) {
 // (1024 threads: 128 VGPRs; one workgroup per CU at the full LDS)
 template <bool GEN>
 __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) {
+  // (the same answer for every wave of the workgroup: this kernel raises its
+  // own flags in the second word, which k_chain_stop passes on after it)
+  if (overflowed(B)) return;
   __shared__ int s_next, s_ncand, s_wsum[2][16];
-  if (block_overflowed(B, &s_ncand)) return;
   __shared__ double s_red[16][NCOL];
   int* const ws0 = s_wsum[0];
   int* const ws1 = s_wsum[1];
@@ -667,7 +669,7 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
   S.n = uni(A.packed ? B.bo_old[ob + Nb] - op0 : A.nops[c]);
   S.m = uni(A.packed ? B.soff_old[os + N] - nd0 : A.nnodes[c]);
   if (S.n > P.blk_opcap || S.m > P.blk_nodecap) {  // (the tables below are sized for the region)
-    if (tid == 0) atomicOr(B.flags, S.n > P.blk_opcap ? FLAG_OP_OVERFLOW : FLAG_NODE_OVERFLOW);
+    if (tid == 0) atomicOr(B.flags + 1, S.n > P.blk_opcap ? FLAG_OP_OVERFLOW : FLAG_NODE_OVERFLOW);
     return;
   }
   for (int b = tid; b < Nb; b += T) S.bo[b] = B.bo_old[ob + b] - op0;
@@ -767,7 +769,7 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
       // The offsets of the launch's earlier sweeps are not written out and
       // the host takes the next arrays for the configuration: none is whole
       // from here on, and the host gives none out (Batch::config_lost)
-      if (tid == 0) atomicOr(B.flags, n > P.blk_opcap ? FLAG_OP_OVERFLOW : FLAG_NODE_OVERFLOW);
+      if (tid == 0) atomicOr(B.flags + 1, n > P.blk_opcap ? FLAG_OP_OVERFLOW : FLAG_NODE_OVERFLOW);
       return;
     }
     for (int s = tid; s < N; s += T) {
@@ -1144,6 +1146,11 @@ __global__ void __launch_bounds__(1024) k_chain_sweeps(DevBatch B, BlockArgs A) 
   }
 }
 
+// What a launch of k_chain_sweeps raised stops the launches after it.
+__global__ void k_chain_stop(DevBatch B) {
+  if (B.flags[1]) B.flags[0] |= B.flags[1];
+}
+
 // Packed form of a batch whose chains stand in regions of their own: chain c's
 // operators to op_base[c], its segments to node_base[c], into the other
 // configuration's arrays; the batch's last chain closes the offsets.
@@ -1208,6 +1215,8 @@ void launch_pack(const DevBatch& B, const int* nops, const int* nnodes, const in
                  hipStream_t st) {
   hipLaunchKernelGGL(k_pack, dim3(B.nchains), dim3(256), 0, st, B, nops, nnodes, op_base, node_base);
 }
+
+void launch_chain_stop(const DevBatch& B, hipStream_t st) { hipLaunchKernelGGL(k_chain_stop, dim3(1), dim3(1), 0, st, B); }
 
 void launch_chain_sweeps(const DevBatch& B, const BlockArgs& A, bool general, int threads, hipStream_t st) {
   if (general) hipLaunchKernelGGL(k_chain_sweeps<true>, dim3(A.grid), dim3(threads), A.lds, st, B, A);

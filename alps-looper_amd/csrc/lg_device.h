@@ -15,16 +15,6 @@ __device__ __forceinline__ bool overflowed(const DevBatch& B) {
   return __hip_atomic_load(B.flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
 }
 
-// The same answer for every thread of the workgroup (word: its own, in LDS).
-// In a launch whose own workgroups set the flag, a workgroup that starts
-// meanwhile could read it with some waves before and some after: those that
-// stay would go on with the tables of those that left unwritten.
-__device__ __forceinline__ bool block_overflowed(const DevBatch& B, int* word) {
-  if (threadIdx.x == 0) *word = overflowed(B);
-  __syncthreads();
-  return *word != 0;
-}
-
 // one thread, in the kernel before a scan: clear the ticket, next epoch
 // (never 0, the value of freshly cleared status words)
 __device__ __forceinline__ void scan_advance_epoch(const DevBatch& B) {

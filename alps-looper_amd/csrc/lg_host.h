@@ -156,7 +156,11 @@ class Batch {
   int capture(int from);
   int check_flags();
   int flags_error() const;
-  void see_flags(int f) { flags_seen = f; config_lost = config_lost || f != 0; }
+  void see_flags(const int* f) {
+    flags_seen = f[0] | f[1];
+    config_lost = config_lost || flags_seen != 0;
+    blk_unseen = false;
+  }
   int config_error() const { return config_lost ? flags_error() : LG_OK; }
   void choose_tiles();
   bool plan_block(std::vector<ChainDev>& ds, long long region, long long op_room, long long node_room);
@@ -205,6 +209,7 @@ class Batch {
   unsigned char* cfg_host = nullptr;              // pinned memory for a configuration on its way out
   static constexpr size_t CFG_HOST_BYTES = 256 << 10;
   int flags_seen = 0;                             // the error flags as last read
+  bool blk_unseen = false;                        // a launch of k_chain_sweeps may have raised flags since
   bool config_lost = false;                       // a sweep overflowed: neither state holds a whole configuration
   std::vector<long long> known_ops;               // operators per chain, while the last records tell them
   int* ring_pos = nullptr;

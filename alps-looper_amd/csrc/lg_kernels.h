@@ -57,7 +57,7 @@ struct DevBatch {
   int* scan_ctl;                    // [0] chunk ticket, [1] launch epoch
   double* col_part;            // [collector terms][chunks] collector partial sums, the chunks of the sweep's segments consecutive
   int* totals;                 // [0] operators, [1] nodes of the new configuration
-  int* flags;
+  int* flags;                  // [0] error flags, [1] those raised by k_chain_sweeps since
   uint32_t* sweep;             // [nchains]
   double* rec_acc;             // [nchains][R_COUNT]
   double* rec_ring;            // [ring][nchains][R_COUNT]
@@ -157,6 +157,7 @@ int block_prepare();                          // 1 when the device grants that m
 int block_lds_least(const ChainDev& d);       // the least that serves any configuration of a chain's region
 int block_lds_for(const ChainDev& d, int n);  // with n operators, every step's arrays at once
 void launch_chain_sweeps(const DevBatch& B, const BlockArgs& A, bool general, int threads, hipStream_t st);
+void launch_chain_stop(const DevBatch& B, hipStream_t st);
 void launch_pack(const DevBatch& B, const int* nops, const int* nnodes, const int* op_base, const int* node_base,
                  hipStream_t st);
 void launch_exchange(const DevBatch& B, hipStream_t st);

@@ -461,8 +461,9 @@ template <int ITEMS>
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan(DevBatch B) {
   constexpr int CHUNK = ITEMS * SCAN_THREADS;
   __shared__ int s_ticket, s_excl;
-  // (one thread decides for the workgroup, as in block_overflowed: the last
-  // bond chunk may set the flag while a site chunk starts)
+  // (one thread decides for the workgroup: the last bond chunk may set the flag
+  // while a site chunk starts, whose other waves would go on without the
+  // ticket of one that left)
   if (threadIdx.x == 0) s_ticket = overflowed(B) ? -1 : atomicAdd(B.scan_ctl, 1);
   __syncthreads();
   const int t = s_ticket;
@@ -2064,6 +2065,10 @@ __global__ void __launch_bounds__(END_THREADS) k_end_sweep(DevBatch B) {
 // the exchange key; log is det_log, so the host reproduces every decision.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_exchange(DevBatch B) {
+  if (B.blk_nops && B.flags[1]) {  // (k_chain_stop; nothing raises a flag meanwhile)
+    if (threadIdx.x == 0) B.flags[0] |= B.flags[1];
+    return;
+  }
   if (overflowed(B)) return;
   const uint32_t step = *B.xstep;
   for (int t = (int)(step & 1) + 2 * (int)threadIdx.x; t + 1 < B.nslots; t += 2 * (int)blockDim.x) {
