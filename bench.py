@@ -6,10 +6,11 @@ latency), one JSON line:
 
 * batched temperature scan: 512 independent chains of the S=1/2 Heisenberg
   antiferromagnet on the 32x32 periodic square lattice, J=1,
-  T_i = 0.05 * 40^(i/511), chain i keyed (23125, i), all chains packed into
-  one launch per sweep stage, the sweep replayed from a captured HIP graph
-  with launch settings chosen by the autotuner.  A "step" is one batched
-  sweep of all 512 chains.  Before the --warmup steps the batch is
+  T_i = 0.05 * 40^(i/511), chain i keyed (23125, i), all chains in one batch,
+  in the form that the autotuner finds the faster: one workgroup per chain
+  with several sweeps a launch, or one launch per sweep stage for all chains,
+  replayed from a captured HIP graph (the line's config says which).  A
+  "step" is one batched sweep of all 512 chains.  Before the --warmup steps the batch is
   equilibrated internally (--equilibrate sweeps from the all-up, empty
   operator string start, whatever --warmup is passed; stated in the output).
   `value` = sum over the timed sweeps and chains of the operator count after
@@ -341,11 +342,17 @@ def scan_params(lg, n=512, L=32):
     return [lg.params(lg.SQUARE, L, 1.0 / T, 1.0, 1.0, seed=SEED, chain_id=i) for i, T in enumerate(scan_temps(n))]
 
 
+def sweep_form(prof, launch):
+    """how the profiled sweeps of a tuned batch ran, and the launch settings they used"""
+    if prof["chain_sweep"] > 0:
+        return "one workgroup per chain, several sweeps a launch", {"form": "one workgroup per chain"}
+    return "one launch per stage for all chains, HIP-graph sweep, autotuned launch settings", launch
+
+
 def run_scan(args, lg):
     plist = scan_params(lg)
     equil = args.equilibrate if args.equilibrate is not None else 400
-    # plain path first: the same chains one chain (and one launch per stage)
-    # at a time -- every 8th chain of the scan, equilibrated like the batch --
+    # plain path first: the same chains one chain at a time -- every 8th chain of the scan, equilibrated like the batch --
     # so that the batch's profiled sweeps are the workload's last launches
     sub = plist[::8]
     plain_sweeps = 20
@@ -380,7 +387,7 @@ def run_scan(args, lg):
     nop_total = float(rec[:, :, 0].sum())
     batched = nop_total / dt
     nop_sweep = nop_total / args.steps
-    # sustained rate over a longer stretch (the same graph replay)
+    # sustained rate over a longer stretch
     sustained = None
     if args.sustain > 0:
         log("scan: sustained %d batched sweeps" % args.sustain)
@@ -390,9 +397,9 @@ def run_scan(args, lg):
     log("scan: profile %d sweeps" % args.profile_sweeps)
     prof = b.profile(args.profile_sweeps)
     launch = b.launch()
+    form, launch_used = sweep_form(prof, launch)
     cfg = {"workload": "512-chain temperature scan: S=1/2 Heisenberg AF on the 32x32 periodic square lattice, "
-                       "J=1, T_i=0.05*40^(i/511), chain i keyed (23125, i); batched (one launch per stage for all "
-                       "chains), HIP-graph sweep, autotuned launch settings",
+                       "J=1, T_i=0.05*40^(i/511), chain i keyed (23125, i); batched: " + form,
            "lattice": "square lattice", "L": 32, "chains": len(plist), "T_min": 0.05, "T_max": 2.0,
            "step": "1 batched sweep of all 512 chains", "seed": SEED}
     out = base_line(args, batched, 1e3 * dt / args.steps, cfg)
@@ -406,7 +413,7 @@ def run_scan(args, lg):
                         "one chain per launch, %.3f s" % (len(sub), plain_sweeps, equil, tp),
         "sustained_value": sustained, "sustained_sweeps": args.sustain,
         "energy_density_coldest_hottest": [float(E[0]), float(E[-1])],
-        "launch": launch,
+        "launch": launch_used,
         "kernel_ms": prof,
         "stages": stage_gbs(prof, nop_sweep, launch["compress"], launch["link"]),
         "sweep_hbm_frac": batched * SWEEP_BYTES_PER_OP / (HBM_PEAK_GBS * 1e9),
