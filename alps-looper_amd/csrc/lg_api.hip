@@ -249,9 +249,10 @@ static double expected_ops(const lg_params& p, const ChainDev& d) {
 
 // Time of a sweep (us): a chain in one workgroup, and a batch on the flat
 // kernels.  Fitted to chains of 41 to 24000 operators on 16 to 3072 bonds
-// (one workgroup: 18 us at 41 operators, 22 at 450, 65 at 3000 on 512 bonds,
-// 40 at 350 on 2048, 540 at 24000 on 2048, where the clusters' accumulators
-// take several passes) and on the flat kernels' launches (60 us at 900
+// (one workgroup, measured and the fit: 20 and 15 us at 53 operators, 27 and
+// 22 at 480, 61 and 58 at 2350 on 512 bonds, 46 and 48 at 1270 on 1152, 570
+// and 543 at 24000 on 2048, where the clusters' accumulators take several
+// passes; the low end is far from the line) and on the flat kernels' launches (60 us at 900
 // operators, 73 at 8900, 131 with virtual sites, 1030 at 3.2M in 512 chains).
 // Near the line, one workgroup and the launches: chain L=64, beta=70 69 and 76
 // us; square 32^2, beta=2.5 67 and 68; S=1 chain L=64, beta=30 111 and 145;
@@ -723,16 +724,21 @@ int Batch::set_layout(std::vector<ChainDev>& ds, const std::vector<uint64_t>& sw
 // for a CU's LDS (both kernels at square 128^2, beta=128: 10000 segments 125
 // us, 15000 107, 20000 100; square 256^2, beta=256: 611, 578, 659).
 void Batch::choose_tiles() {
-  // segments of a site: expected, and at most (an operator's weight is the
-  // bond's offset less its energy); the replicas of an exchange come to every
-  // temperature
+  // segments of a site: expected, and at most; the replicas of an exchange
+  // come to every temperature.  A bond holds beta (offset - its energy)
+  // operators in the mean, and the energy is at least -|Jz|/4 - e |Jxy|: the
+  // ground states of the two parts apart.  e is the XY ring's energy per bond,
+  // 1 / (L sin(pi / L)), which falls to 1/pi = 0.318; rings of 6 to 16 sites
+  // have up to 0.333, within the margin that set_tiles adds (a tile beyond its
+  // LDS unites in memory), 2 and 4 sites 0.5 and 0.354
   std::vector<double> mean, most;
   double segs = 0, mean_max = 0, most_max = 0;
   for (size_t c = 0; c < chains.size(); ++c) {
     const ChainDev& d = chains[c];
     const lg_params& p = params[c];
     mean.push_back(2 * expected_ops(p, d) / d.N);
-most.push_back(2 * d.beta / d.N * (d.offset_total + d.nb_real * (std::fabs(p.jz) / 4 + (d.L > 4 ? 0.32 : 0.5) * std::fabs(p.jxy))));
+    most.push_back(2 * d.beta / d.N *
+                   (d.offset_total + d.nb_real * (std::fabs(p.jz) / 4 + (d.L > 4 ? 0.32 : 0.5) * std::fabs(p.jxy))));
     segs += mean[c] * d.N;
     mean_max = std::max(mean_max, mean[c]);
     most_max = std::max(most_max, most[c]);

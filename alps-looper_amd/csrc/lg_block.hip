@@ -603,11 +603,12 @@ __device__ __forceinline__ void seg_winding(int fl, int flo, int& d0, int& d1) {
 
 }  // namespace
 
-// Bound by the instructions of one CU (110000 wave instructions a sweep at 3000
-// operators, 46 of 67 us), so the steps hold little per operator; 256, 512 or
+// Bound by the instructions of one CU (80000 vector instructions a sweep at
+// 2400 operators, which the CU's four SIMDs issue in 33 of 61 us; the rest is
+// barriers, LDS and loads), so the steps hold little per operator; 256, 512 or
 // 1024 threads by the operators, as few as keep a step's loads in flight, so
 // that small chains share a CU.  A sweep of 450 operators: 65 us in eight
-// launches, 30 here; 512 chains of up to 24000 operators: 1.30 and 0.59 ms,
+// launches, 27 here; 512 chains of up to 24000 operators: 1.30 and 0.59 ms,
 // the largest chain's time (link 116 us, unions 98, estimator 115, draws 64,
 // tests 46, places 75 of it).
 // GEN: virtual sites (S > 1/2), in-site bonds (single-ion term) or site

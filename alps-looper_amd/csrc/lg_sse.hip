@@ -49,7 +49,7 @@ __device__ __forceinline__ int with_lane(int v, int l, int x) { return lane_id()
 // its graph; the operators, the spins and the string follow for all lanes at
 // once when the next 64 steps or operators come in.  One step at a time with
 // words, sites and spins from LDS took 280 ns a step (16.7 ms for the coldest
-// of 512 chains of 32^2, about 50000 steps); runs with every emitted
+// of 512 chains of 32^2, about 60000 steps); runs with every emitted
 // operator stored in the loop 8.9 ms.
 __global__ void __launch_bounds__(SSE_THREADS) k_sse_walk(DevBatch B) {
   if (blockIdx.x == 0 && threadIdx.x == 0) scan_advance_epoch(B);  // for k_scan, which follows
