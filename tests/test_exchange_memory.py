@@ -2,6 +2,7 @@
 for every replica only where one workgroup sweeps each."""
 
 import ctypes
+import gc
 import math
 
 import pytest
@@ -17,6 +18,7 @@ def _taken(make):
         assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
         return free.value
 
+    gc.collect()  # (handles that earlier tests left)
     before = now()
     x = make()
     after = now()
